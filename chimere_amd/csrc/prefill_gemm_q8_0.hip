@@ -1,0 +1,6 @@
+// prefill_gemm_q8_0.hip -- the prefill chunk's expert launches, Q8_0 experts.
+#include "prefill_gemm.h"
+
+namespace chimere {
+template void pf_launch_experts<T_Q8_0>(const PfArgs&, int, hipStream_t);
+}  // namespace chimere

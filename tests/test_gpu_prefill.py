@@ -219,3 +219,43 @@ def test_prefill_model_layer_types_full_shape(dev):
     layer = kq_layer(dev, 880, O.IQ3_S, O.Q5_K, 2048, 512, 256, 8)
     g = torch.Generator(device=dev).manual_seed(88)
     prefill_check(layer, torch.randn(96, 2048, generator=g, device=dev))
+
+
+@pytest.mark.parametrize("et", [O.Q4_0, O.Q8_0, O.IQ3_S])
+@pytest.mark.parametrize("st", [None, O.Q4_0, O.Q8_0, O.IQ3_S, O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("H,F,E,K,T", [
+    (256, 256, 16, 1, 11),     # one K chunk; tiles of 16 pairs
+    (768, 512, 8, 2, 33),      # three gate/up chunks, two down chunks; tiles of 32, one of a single pair (shared)
+    (768, 256, 4, 2, 130),     # tiles of 64: full ones, short ones, one of 2 (shared)
+])
+def test_prefill_tile_sizes(dev, et, st, H, F, E, K, T):
+    """Every expert x shared type at the three tile sizes (chosen by the
+    average pairs per expert), odd and even numbers of K chunks, full and
+    short tiles: bit-exact against the oracle's L=1 order."""
+    print(f"prefill tiles et={et} st={st} H={H} F={F} E={E} K={K} T={T}", flush=True)
+    if st in (O.Q4_K, O.Q5_K, O.Q6_K):
+        layer = kq_layer(dev, 900 + et + st + T, et, st, H, F, E, K)
+    else:
+        layer = build(dev, 900 + et + (st or 0) + T, H=H, F=F, E=E, K=K, et=et, st=st, gate_vec=st is not None)
+    g = torch.Generator(device=dev).manual_seed(T + et)
+    prefill_check(layer, torch.randn(T, H, generator=g, device=dev))
+
+
+@pytest.mark.parametrize("et", [O.Q4_0, O.Q8_0, O.IQ3_S])
+@pytest.mark.parametrize("off", [2, 4, 14])
+def test_prefill_weight_offsets(dev, et, off):
+    """Expert tensors that start at any even address (a chunk then begins
+    inside a 16-byte granule, the words of a block at either phase) give the
+    bits of aligned ones."""
+    print(f"prefill offsets et={et} off={off}", flush=True)
+    layer = build(dev, 950 + et, H=512, F=256, E=8, K=2, et=et, st=et)
+    g = torch.Generator(device=dev).manual_seed(off)
+    x = torch.randn(40, 512, generator=g, device=dev)
+    want = host(layer.prefill(x))
+    moved = []
+    for t in layer.tensors[1:4]:
+        buf = torch.zeros(t.numel() + 32, dtype=torch.uint8, device=dev)
+        buf[off:off + t.numel()] = t.reshape(-1)
+        moved.append(buf[off:off + t.numel()].view(t.shape))
+    other = MoeLayer(layer.tensors[0], *moved, et, 2, shared=layer.tensors[6:9], shared_type=et)
+    assert (host(other.prefill(x)).view(np.uint32) == want.view(np.uint32)).all()
