@@ -130,9 +130,10 @@ __global__ __launch_bounds__(256) void k_pf_quant(PfArgs a) {
     const float xi = a.x[t * a.H + b * QK + i];
     const float amax = bfly32_max(__builtin_fabsf(xi));
     const float d = amax / 127.0f;
-    const float qv = amax == 0.0f ? 0.0f : __builtin_roundf(xi / d);
-    a.xh[(t * nb + b) * QK + i] = (_Float16)(int)qv;
-    const float sq = bfly32_sum(qv);   // exact: integers below 2^12
+    // (int8_t): where d underflows to 0 the byte the Q8_1 block would hold
+    const int qv = amax == 0.0f ? 0 : (int8_t)(int)__builtin_roundf(xi / d);
+    a.xh[(t * nb + b) * QK + i] = (_Float16)qv;
+    const float sq = bfly32_sum((float)qv);   // exact: integers below 2^12
     if (i == 0) {
         a.xd[t * nb + b] = f2h(d);
         a.xs[t * nb + b] = sq;

@@ -659,10 +659,11 @@ __global__ __launch_bounds__(PF_THREADS, 2) void k_pf_gate_up(PfArgs a) {
                 for (int i = 0; i < 4; i++) {
                     const int p = 16 * m + 4 * q + i;
                     const float amax = __builtin_fmaxf(am[m][i], ov[i]), d = amax / 127.0f;
-                    const float qv = amax == 0.0f ? 0.0f : __builtin_roundf(acc[0][m][i] / d);
-                    acc[1][m][i] = qv;
+                    // (int8_t): where d underflows to 0 the byte the Q8_1 block would hold
+                    const int qv = amax == 0.0f ? 0 : (int8_t)(int)__builtin_roundf(acc[0][m][i] / d);
+                    acc[1][m][i] = (float)qv;
                     if (p < np) {
-                        a.hh[(int64_t)(start + p) * a.F + f0 + 16 * wave + c] = (_Float16)(int)qv;
+                        a.hh[(int64_t)(start + p) * a.F + f0 + 16 * wave + c] = (_Float16)qv;
                         if (c == 0 && (wave & 1) == 0) a.hd[(start + p) * nb + (f0 >> 5) + (wave >> 1)] = f2h(d);
                     }
                 }

@@ -259,3 +259,17 @@ def test_prefill_weight_offsets(dev, et, off):
         moved.append(buf[off:off + t.numel()].view(t.shape))
     other = MoeLayer(layer.tensors[0], *moved, et, 2, shared=layer.tensors[6:9], shared_type=et)
     assert (host(other.prefill(x)).view(np.uint32) == want.view(np.uint32)).all()
+
+
+def test_prefill_subnormal_activations(dev):
+    """Tokens so small that a Q8_1 block's scale is subnormal or zero, and
+    weight scales below the smallest normal f16: bit-exact against the oracle."""
+    layer = build(dev, 960, H=512, F=256, E=8, K=2)
+    for m in layer.tensors[1:4]:
+        b = m.view(-1, 18)
+        b[::3, 0], b[::3, 1] = 0x7, 0x1             # d = 263 * 2^-24
+    g = torch.Generator(device=dev).manual_seed(6)
+    x = torch.randn(24, 512, generator=g, device=dev)
+    for i, s in enumerate((1e-38, 1e-41, 1e-43, 3e-45, 1e-6)):
+        x[3 * i] *= s
+    prefill_check(layer, x, margin=False)
