@@ -28,7 +28,18 @@ struct MmvqArgs {
     int64_t w_slot_stride;  // bytes per expert
     int64_t x_slot_stride;  // bytes between slots' inputs (0: shared)
     int64_t y_slot_stride;  // floats between slots' outputs
+    // f32 entry points, one launch: x is the f32 row; the first work-group
+    // leaves its Q8_1 blocks, zero blocks up to raw_blocks, in raw
+    uint8_t* raw;
+    int raw_blocks;
 };
+
+// The zero blocks past the row's own in the caller's Q8_1 scratch
+__device__ __forceinline__ void raw_padding(const MmvqArgs& a) {
+    uint32_t* o = (uint32_t*)a.raw;
+    for (int i = a.ncols / QK * (Q8_1_BYTES / 4) + threadIdx.x; i < a.raw_blocks * (Q8_1_BYTES / 4); i += GEMV_THREADS)
+        o[i] = 0;
+}
 
 // Blocks per K chunk of the GEMV tile: 64 for every type, which puts a
 // 2048-column Q8_0 row in one chunk (one exposed round trip per work-group
@@ -44,7 +55,8 @@ constexpr int MMVQ_BLOCKS = 64;
 template <int T>
 constexpr int mmvq_pad() { return T == T_Q4_0 || T == T_Q4_0S || T == T_Q8_0 ? 48 : (T == T_IQ3_S ? 80 : 0); }
 
-template <int T, int NTOK>
+// XF32: the f32 entry points' row, quantized by every work-group for itself
+template <int T, int NTOK, bool XF32 = false>
 __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq(MmvqArgs a) {
     constexpr int CBLK = MMVQ_BLOCKS;
     constexpr int CB = chunk_bytes<T>(CBLK), PAD = mmvq_pad<T>();
@@ -62,11 +74,16 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq(MmvqArgs a) {
     if constexpr (T == T_IQ3_S)
         for (int i = tid; i < 512; i += GEMV_THREADS) grid[i] = c_iq3s_grid_mmvq[i];
 
+    uint8_t* raw = nullptr;
+    if (XF32 && blockIdx.x == 0) {
+        raw = a.raw;
+        raw_padding(a);
+    }
     float acc[1][NTOK];
-    tile_gemv<T, NTOK, TILE_ROWS, 1, CBLK, CPOL_STREAM, PAD, true>(tile, &xs[0][0], grid,
+    tile_gemv<T, NTOK, TILE_ROWS, 1, CBLK, CPOL_STREAM, PAD, true, XF32>(tile, &xs[0][0], grid,
                                      a.W + e * a.w_slot_stride + (int64_t)r0 * rb, nr,
                                      nullptr, 0, rb, a.ncols, a.x + slot * a.x_slot_stride, a.x_tok_stride,
-                                     nullptr, a.ntok, acc);
+                                     nullptr, a.ntok, acc, raw);
     if (g < nr) {
 #pragma unroll
         for (int t = 0; t < NTOK; t++) {
@@ -84,12 +101,12 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq(MmvqArgs a) {
 // compile-time chunk count (the same fp32 order as tile_gemv; the general
 // path's run-time row count and chunk loop cost ~0.35 us of latency per
 // launch: Q8_0 4096x2048 4.24 -> 3.90 us, Q4_0 head 30.8 -> 28.6 us).
-template <int T, int NCH>
+template <int T, int NCH, bool XF32 = false>
 __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_nc(MmvqArgs a) {
     constexpr int CBLK = MMVQ_BLOCKS, CB = chunk_bytes<T>(CBLK), LS = CB + mmvq_pad<T>();
     static_assert(CB % 16 == 0, "16-byte pieces");
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE_ROWS * LS + 16];
-    __shared__ XLds xs[CBLK];
+    __shared__ XLds xs[XF32 ? NCH * CBLK : CBLK];
     __shared__ uint32_t grid[T == T_IQ3_S ? 512 : 1];
     const int tid = threadIdx.x, g = tid >> 4, j = tid & 15;
     const int slot = blockIdx.y;
@@ -105,7 +122,12 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_nc(MmvqArgs a) {
         if (c > 0) __syncthreads();   // every wave is done with the previous chunk
         stage_rows_fixed<CB, LS, 16, TILE_ROWS, GEMV_THREADS, CPOL_STREAM, true>(tile, W + c * CB, TILE_ROWS, nullptr,
                                                                                   RB, TILE_ROWS, tid);
-        if (tid < CBLK) {
+        if constexpr (XF32) {
+            if (c == 0) {   // the whole row, under the first chunk's copies
+                quant_xlds<GEMV_THREADS>((const float*)X, 0, NCH * CBLK, xs, blockIdx.x == 0 ? a.raw : nullptr);
+                if (blockIdx.x == 0) raw_padding(a);
+            }
+        } else if (tid < CBLK) {
             XBlk xb;
             load_xblk(X + (int64_t)(c * CBLK + tid) * Q8_1_BYTES, xb);
             XLds& o = xs[tid];
@@ -119,7 +141,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_nc(MmvqArgs a) {
 #pragma unroll 1
         for (int b = j; b < CBLK; b += SLOTS) {
             XBlk xb;
-            xlds_to_blk(xs[b], xb);
+            xlds_to_blk(xs[XF32 ? c * CBLK + b : b], xb);
             WBlk wb;
             block_decode<T>(tile + g * LS, b, grid, wb);
             acc = wacc<T>(wb, xb, acc);
@@ -129,23 +151,40 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_nc(MmvqArgs a) {
     if (j == 0) a.y[slot * a.y_slot_stride + blockIdx.x * TILE_ROWS + g] = v;
 }
 
-template <int T>
+template <int T, bool XF32 = false>
 static void launch_t(const MmvqArgs& a, int nslots, hipStream_t s) {
     dim3 grid((unsigned)((a.nrows + TILE_ROWS - 1) / TILE_ROWS), (unsigned)nslots);
     if constexpr (chunk_bytes<T>(MMVQ_BLOCKS) % 16 == 0) {
         const int nch = a.ncols / (MMVQ_BLOCKS * QK);
         if (a.ntok == 1 && a.ncols % (MMVQ_BLOCKS * QK) == 0 && (nch == 1 || nch == 2) && a.nrows % TILE_ROWS == 0 &&
             (((uintptr_t)a.W | (uintptr_t)a.w_slot_stride) & 15) == 0) {
-            if (nch == 1) hipLaunchKernelGGL((k_mmvq_nc<T, 1>), grid, dim3(GEMV_THREADS), 0, s, a);
-            else hipLaunchKernelGGL((k_mmvq_nc<T, 2>), grid, dim3(GEMV_THREADS), 0, s, a);
+            if (nch == 1) hipLaunchKernelGGL((k_mmvq_nc<T, 1, XF32>), grid, dim3(GEMV_THREADS), 0, s, a);
+            else hipLaunchKernelGGL((k_mmvq_nc<T, 2, XF32>), grid, dim3(GEMV_THREADS), 0, s, a);
             return;
         }
     }
     dim3 blk(GEMV_THREADS);
+    if constexpr (XF32) {
+        hipLaunchKernelGGL((k_mmvq<T, 1, true>), grid, blk, 0, s, a);
+        return;
+    }
     switch (a.ntok) {
 #define CASE(N) case N: hipLaunchKernelGGL((k_mmvq<T, N>), grid, blk, 0, s, a); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
+    }
+}
+
+// f32 activation row: x, raw and raw_blocks of a set (k_mmvq)
+static void launch_mmvq_f32(int type, const MmvqArgs& a, hipStream_t s) {
+    switch (type) {
+    case T_Q8_0: launch_t<T_Q8_0, true>(a, 1, s); break;
+    case T_Q4_0: launch_t<T_Q4_0, true>(a, 1, s); break;
+    case T_IQ3_S: launch_t<T_IQ3_S, true>(a, 1, s); break;
+    case T_Q4_K: launch_t<T_Q4_K, true>(a, 1, s); break;
+    case T_Q5_K: launch_t<T_Q5_K, true>(a, 1, s); break;
+    case T_Q6_K: launch_t<T_Q6_K, true>(a, 1, s); break;
+    case T_MXFP4: launch_t<T_MXFP4, true>(a, 1, s); break;
     }
 }
 
@@ -195,9 +234,22 @@ static void gemv_entry(const char* who, int type, const void* W, const void* x, 
     // the s-form GEMV reads plain Q4_0 blocks
     if (!check_gemv(who, type == T_Q4_0S ? T_Q4_0 : type, W, x, y, ncols, nrows, nrows_y_padded, ntok)) return;
     MmvqArgs a{(const uint8_t*)W, (const uint8_t*)x, y, ncols, nrows, ntok,
-               (int64_t)nrows_y_padded * Q8_1_BYTES, nrows, nullptr, 0, 0, 0};
+               (int64_t)nrows_y_padded * Q8_1_BYTES, nrows, nullptr, 0, 0, 0, nullptr, 0};
     launch_mmvq(type, a, 1, s);
     check_launch(who);
+}
+
+// One launch for an f32 activation row (every work-group quantizes it for
+// itself while its first weights are in flight) instead of a quantizer launch
+// and the GEMV: the launch costs 1.1-1.4 us per call, the quantizing about
+// 0.25 us of vector-ALU time per work-group and 2048 columns.  HIP graph, two
+// launches / one: Q8_0 4096x2048 (256 work-groups) 5.4 / 4.5 us, Q5_K 5.4 /
+// 4.3; 16384x2048 (1024) Q8_0 10.2 / 9.0, Q4_0 7.9 / 7.1; 65536x2048 (4096)
+// Q4_0 16.1 / 17.7; 8192x4096 (512, two chunks) Q5_K 9.5 / 8.8; 16384x4096
+// (1024, two chunks) Q5_K 12.2 / 13.1.
+static bool f32_one_launch(const float* x, int ncols, int nrows) {
+    const int64_t wg = (nrows + TILE_ROWS - 1) / TILE_ROWS, chunks = (ncols + MMVQ_BLOCKS * QK - 1) / (MMVQ_BLOCKS * QK);
+    return ((uintptr_t)x & 15) == 0 && wg * chunks <= 1024;   // 16-byte loads of x
 }
 
 static void gemv_f32_entry(const char* who, int type, const void* W, const float* x, float* y,
@@ -208,6 +260,13 @@ static void gemv_f32_entry(const char* who, int type, const void* W, const float
         return;
     }
     if (!check_gemv(who, type, W, scratch, y, ncols, nrows, ncols_padded / 32, 1)) return;
+    if (f32_one_launch(x, ncols, nrows)) {
+        MmvqArgs a{(const uint8_t*)W, (const uint8_t*)x, y, ncols, nrows, 1, 0, nrows, nullptr, 0, 0, 0,
+                   (uint8_t*)scratch, ncols_padded / 32};
+        launch_mmvq_f32(type, a, s);
+        check_launch(who);
+        return;
+    }
     launch_quantize_q8_1(x, scratch, ncols, ncols_padded, 1, s);
     gemv_entry(who, type, W, scratch, y, ncols, nrows, ncols_padded / 32, 1, s);
 }
@@ -224,7 +283,7 @@ static void gemv_batched_entry(const char* who, int type, const void* W, const v
         return;
     }
     MmvqArgs a{(const uint8_t*)W, (const uint8_t*)x, y, ncols, nrows, 1,
-               0, 0, ids, expert_stride, input_stride, nrows};
+               0, 0, ids, expert_stride, input_stride, nrows, nullptr, 0};
     launch_mmvq(type, a, top_k, s);
     check_launch(who);
 }

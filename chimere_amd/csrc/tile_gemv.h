@@ -50,6 +50,61 @@ __device__ __forceinline__ void xlds_to_blk(const XLds& s, XBlk& x) {
     x.sumq = s.sumq;
 }
 
+// Blocks [b0, b0 + cb) of an f32 row (16-byte aligned) quantized to Q8_1 into
+// xs[0 .. cb): the values of k_quantize_q8_1, four lanes per block with eight
+// elements each.  raw (not null): the blocks are written there too.  NTH
+// threads, a multiple of 64; lanes past the last block repeat it.
+template <int NTH>
+__device__ __forceinline__ void quant_xlds(const float* __restrict__ x, int b0, int cb, XLds* __restrict__ xs,
+                                           uint8_t* __restrict__ raw) {
+    for (int i0 = 0; i0 < 4 * cb; i0 += NTH) {
+        const int i = i0 + (int)threadIdx.x, b = min(i >> 2, cb - 1), sub = i & 3;
+        const float4 u0 = *(const float4*)(x + (int64_t)(b0 + b) * QK + 8 * sub);
+        const float4 u1 = *(const float4*)(x + (int64_t)(b0 + b) * QK + 8 * sub + 4);
+        float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+        float amax = __builtin_fabsf(v[0]);
+#pragma unroll
+        for (int k = 1; k < 8; k++) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[k]));
+        amax = __builtin_fmaxf(amax, xlane<2>(amax));
+        amax = __builtin_fmaxf(amax, xlane<1>(amax));
+        const float d = amax / 127.0f;
+        uint32_t w[2] = {0, 0};
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int q = amax == 0.0f ? 0 : (int)__builtin_roundf(v[k] / d);
+            w[k >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (k & 3));
+        }
+        int sq = dot4((int)w[0], 0x01010101, dot4((int)w[1], 0x01010101, 0));
+        sq += xlane<2>(sq);
+        sq += xlane<1>(sq);
+        const uint32_t dh = f2h(d);
+        if ((i >> 2) < cb) {
+            XLds& o = xs[b];
+            o.q[2 * sub] = (int)w[0];
+            o.q[2 * sub + 1] = (int)w[1];
+            if (sub == 0) { o.d = h2f(dh); o.sumq = sq; }
+        }
+        if (raw) {
+            // the sum of x in the butterfly order (xor 16, 8 across the
+            // block's lanes, 4, 2, 1 inside one)
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = v[k] + xlane<2>(v[k]);
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = v[k] + xlane<1>(v[k]);
+#pragma unroll
+            for (int m = 4; m >= 1; m >>= 1)
+#pragma unroll
+                for (int k = 0; k < m; k++) v[k] = v[k] + v[k + m];
+            if ((i >> 2) < cb) {
+                uint32_t* o = (uint32_t*)(raw + (int64_t)(b0 + b) * Q8_1_BYTES);
+                if (sub == 0) o[0] = dh | (f2h(v[0]) << 16);
+                o[1 + 2 * sub] = w[0];
+                o[2 + 2 * sub] = w[1];
+            }
+        }
+    }
+}
+
 // The dots of one staged chunk: rows [0, nr) of the tile (LDS row stride
 // lseg) against the chunk's cb decoded activation blocks per token.  KC > 0:
 // a full chunk of a compile-time row stride KC and CBLK blocks (the block loop
@@ -106,12 +161,13 @@ __device__ __forceinline__ void tile_compute(const uint8_t* __restrict__ tl, int
 // FAST: a full chunk (cb == CBLK) with 16-byte aligned pieces, staged by
 // stage_rows_fixed (the copies issued back to back) and computed with a
 // compile-time row stride and block count; otherwise the general path.
-template <int T, int NT, int RG, int RPG, int CBLK, int CPOL, int PAD, bool FAST>
+// XF32: X is the f32 row itself (one token), quantized here (xraw: see quant_xlds).
+template <int T, int NT, int RG, int RPG, int CBLK, int CPOL, int PAD, bool FAST, bool XF32 = false>
 __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __restrict__ xs,
                                            const uint32_t* __restrict__ grid, const uint8_t* base1, int n1,
                                            const uint8_t* base2, int n2, int64_t rb, int b0, int cb,
                                            const uint8_t* __restrict__ X, int64_t x_tok_stride, const int* toks,
-                                           int ntok, float (&acc)[RPG][NT]) {
+                                           int ntok, float (&acc)[RPG][NT], uint8_t* xraw = nullptr) {
     constexpr int NTH = RG * SLOTS;
     constexpr int CB = chunk_bytes<T>(CBLK);
     const int tid = threadIdx.x;
@@ -136,7 +192,8 @@ __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __r
         if (n1) stage_rows<stage_dw<T>(), CPOL>(tile, base1 + goff, rb, n1, seg, tid, NTH, lseg);
         if (n2) stage_rows<stage_dw<T>(), CPOL>(tile + n1 * lseg, base2 + goff, rb, n2, seg, tid, NTH, lseg);
     }
-    for (int i = tid; i < ntok * cb; i += NTH) {
+    if constexpr (XF32) quant_xlds<NTH>((const float*)X, b0, cb, xs, xraw);
+    else for (int i = tid; i < ntok * cb; i += NTH) {
         const int t = i / cb, b = i - t * cb;
         const int tk = toks ? toks[t] : t;
         XBlk xb;
@@ -175,14 +232,15 @@ __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __r
 // FIX: full 16-byte aligned chunks on tile_chunk's FAST path (measured
 // faster for the standalone GEMV, slower -- more registers -- in the MoE
 // kernels' tiles)
+// XF32, xraw: the activation row in f32 (tile_chunk)
 template <int T, int NT, int RG, int RPG, int CBLK = ChunkGeom<T>::BLOCKS, int CPOL = 0, int PAD = 0,
-          bool FIX = false>
+          bool FIX = false, bool XF32 = false>
 __device__ __forceinline__ void tile_gemv(uint8_t* __restrict__ tile, XLds* __restrict__ xs,
                                           const uint32_t* __restrict__ grid,
                                           const uint8_t* base1, int n1, const uint8_t* base2, int n2,
                                           int64_t rb, int ncols, const uint8_t* __restrict__ X,
                                           int64_t x_tok_stride, const int* toks, int ntok,
-                                          float (&acc)[RPG][NT]) {
+                                          float (&acc)[RPG][NT], uint8_t* xraw = nullptr) {
     static_assert(CBLK % SLOTS == 0 && (QTraits<T>::ELEMS != 256 || CBLK % 8 == 0) && CBLK <= MAX_CHUNK_BLOCKS, "chunk");
     const int nb = ncols / QK;
 #pragma unroll
@@ -195,12 +253,12 @@ __device__ __forceinline__ void tile_gemv(uint8_t* __restrict__ tile, XLds* __re
     for (int b0 = 0; b0 < nb; b0 += CBLK) {
         // chunk offsets are multiples of the (16-byte multiple) chunk bytes
         if (FIXOK && al16 && nb - b0 >= CBLK)
-            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, FIXOK>(tile, xs, grid, base1, n1, base2, n2, rb, b0, CBLK, X,
-                                                               x_tok_stride, toks, ntok, acc);
+            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, FIXOK, XF32>(tile, xs, grid, base1, n1, base2, n2, rb, b0, CBLK,
+                                                                     X, x_tok_stride, toks, ntok, acc, xraw);
         else
-            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, false>(tile, xs, grid, base1, n1, base2, n2, rb, b0,
-                                                               min(CBLK, nb - b0), X, x_tok_stride, toks, ntok,
-                                                               acc);
+            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, false, XF32>(tile, xs, grid, base1, n1, base2, n2, rb, b0,
+                                                                     min(CBLK, nb - b0), X, x_tok_stride, toks, ntok,
+                                                                     acc, xraw);
     }
 }
 

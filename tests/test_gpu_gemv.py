@@ -270,3 +270,37 @@ def test_gemv_q4_0_sform_bit_exact(dev, nrows, ncols):
     bound = (8 * np.abs(dw) * np.abs(sx - dx * sq)[None, :]).sum(axis=1)
     diff = np.abs(gs.astype(np.float64) - ge)
     assert (diff <= bound + 1e-5 * np.abs(ge).max()).all() and diff.max() > 0
+
+
+@pytest.mark.parametrize("t", [O.Q8_0, O.Q4_0, O.IQ3_S, O.Q4_K, O.Q5_K, O.Q6_K, O.MXFP4])
+@pytest.mark.parametrize("nrows,ncols", [
+    (16, 256), (37, 2048), (64, 4096), (33, 2304), (48, 6144),   # one launch: whole and ragged chunks and tiles
+    (16384, 2048), (16385, 2048), (8192, 4096), (8193, 4096),    # the last one-launch size and the next
+])
+def test_f32_gemv_is_quantizer_plus_gemv(dev, t, nrows, ncols):
+    """The f32 entry points in one launch and in two: the output bits and the
+    scratch bytes (zero blocks up to the padded length included) of the
+    quantizer followed by the Q8_1 entry point; an input that is not 16-byte
+    aligned gives the same."""
+    rng = np.random.default_rng(nrows + ncols + t)
+    w = torch.randint(0, 120, (nrows * O.row_bytes(t, ncols),), dtype=torch.uint8, device=dev,
+                      generator=torch.Generator(device=dev).manual_seed(t))
+    x = rng.standard_normal(ncols).astype(np.float32)
+    x[:32] = 0
+    x[40:50] *= np.float32(1e-44)
+    pad = G.pad(ncols, 512)
+    xq = dev_t(O.quantize_q8_1(x, pad), dev)
+    want = torch.zeros(nrows, device=dev)
+    G.gemv_multi(t, w, xq, want, nrows, ncols, 1)
+    fn = {O.Q8_0: G.ggml_gpu_gemv_q8_0_f32, O.Q4_0: G.ggml_gpu_gemv_q4_0_f32, O.IQ3_S: G.ggml_gpu_gemv_iq3s_f32,
+          O.Q4_K: G.ggml_gpu_gemv_q4k_f32, O.Q5_K: G.ggml_gpu_gemv_q5k_f32, O.Q6_K: G.ggml_gpu_gemv_q6k_f32,
+          O.MXFP4: G.ggml_gpu_gemv_mxfp4_f32}[t]
+    buf = torch.empty(ncols + 4, device=dev)
+    for off in (0, 1):
+        xd = buf[off:off + ncols]
+        xd.copy_(dev_t(x, dev))
+        scratch = torch.full((pad // 32 * 36,), 255, dtype=torch.uint8, device=dev)
+        y = torch.zeros(nrows, device=dev)
+        fn(w, xd, y, scratch, nrows, ncols)
+        assert (host(scratch) == host(xq).reshape(-1)).all()
+        assert (host(y).view(np.uint32) == host(want).view(np.uint32)).all()
