@@ -121,30 +121,84 @@ __global__ __launch_bounds__(256) void k_pf_router(PfArgs a) {
     }
 }
 
-// Q8_1 of x (the values of k_quantize_q8_1: one 32-lane half-wave per block)
-// in the GEMMs' layout.  Grid: (groups of 8 blocks, tokens)
+// Q8_1 of x (the values of k_quantize_q8_1) in the GEMMs' layout, and the
+// expert counts zeroed for k_pf_topk.  Eight lanes per block, 16-byte loads
+// (two half-waves per block with 4-byte loads and 2-byte stores: 4096 tokens
+// 19.7 us).  Grid: groups of 32 blocks of all tokens
 __global__ __launch_bounds__(256) void k_pf_quant(PfArgs a) {
-    const int b = blockIdx.x * 8 + (threadIdx.x >> 5), i = threadIdx.x & 31, nb = a.H / QK;
-    const int64_t t = blockIdx.y;
-    if (b >= nb) return;   // whole half-wave exits together
-    const float xi = a.x[t * a.H + b * QK + i];
-    const float amax = bfly32_max(__builtin_fabsf(xi));
+    if (blockIdx.x == 0)
+        for (int e = threadIdx.x; e < a.E; e += 256) a.cnt[e] = 0;
+    const int64_t b = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+    const int i = threadIdx.x & 7;
+    if (b >= (int64_t)a.T * (a.H / QK)) return;   // whole groups of eight lanes exit together
+    const float* src = a.x + b * QK + 4 * i;
+    float v[4];
+    if (((uintptr_t)a.x & 15) == 0) {
+        const float4 u = *(const float4*)src;
+        v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = src[k];
+    }
+    float amax = __builtin_fabsf(v[0]);
+#pragma unroll
+    for (int k = 1; k < 4; k++) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[k]));
+    amax = __builtin_fmaxf(amax, xlane<4>(amax));
+    amax = __builtin_fmaxf(amax, xlane<2>(amax));
+    amax = __builtin_fmaxf(amax, xlane<1>(amax));
     const float d = amax / 127.0f;
-    // (int8_t): where d underflows to 0 the byte the Q8_1 block would hold
-    const int qv = amax == 0.0f ? 0 : (int8_t)(int)__builtin_roundf(xi / d);
-    a.xh[(t * nb + b) * QK + i] = (_Float16)qv;
-    const float sq = bfly32_sum((float)qv);   // exact: integers below 2^12
+    v4h h;
+    int sq = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        // (int8_t): where d underflows to 0 the byte the Q8_1 block would hold
+        const int q = amax == 0.0f ? 0 : (int8_t)(int)__builtin_roundf(v[k] / d);
+        h[k] = (_Float16)q;
+        sq += q;
+    }
+    sq += xlane<4>(sq);
+    sq += xlane<2>(sq);
+    sq += xlane<1>(sq);
+    *(v4h*)(a.xh + b * QK + 4 * i) = h;
     if (i == 0) {
-        a.xd[t * nb + b] = f2h(d);
-        a.xs[t * nb + b] = sq;
+        a.xd[b] = f2h(d);
+        a.xs[b] = (float)sq;
     }
 }
 
-// P2: one wave per token
-__global__ __launch_bounds__(64) void k_pf_topk(PfArgs a) {
-    __shared__ uint64_t s_tk[128];
-    const int t = blockIdx.x;
-    topk_wave_any(a.logits + (int64_t)t * a.E, a.E, a.K, a.ids + t * a.K, a.wts + t * a.K, s_tk);
+// P2: one wave per token, 16 tokens per work-group; the work-group's pairs are
+// counted per expert in LDS, and one global count per (work-group, expert)
+// gives each pair its rank among its expert's
+constexpr int PF_TKT = 16;
+__global__ __launch_bounds__(64 * PF_TKT) void k_pf_topk(PfArgs a) {
+    __shared__ uint64_t s_tk[PF_TKT][128];
+    __shared__ int s_ids[PF_TKT][MAX_K], cnt[MAX_E];
+    __shared__ float s_w[PF_TKT][MAX_K];
+    const int tid = threadIdx.x, wave = tid >> 6, t = blockIdx.x * PF_TKT + wave;
+    for (int e = tid; e < a.E; e += 64 * PF_TKT) cnt[e] = 0;
+    if (t < a.T) topk_wave_any(a.logits + (int64_t)t * a.E, a.E, a.K, s_ids[wave], s_w[wave], s_tk[wave]);
+    __syncthreads();
+    // thread -> pair of the work-group (16 tokens x at most 16 experts)
+    const int pt = tid / MAX_K, k = tid - pt * MAX_K;
+    const bool on = pt < PF_TKT && k < a.K && blockIdx.x * PF_TKT + pt < a.T;
+    int e = -1, r = 0;
+    if (on) {
+        e = s_ids[pt][k];
+        if ((unsigned)e < (unsigned)a.E) r = atomicAdd(&cnt[e], 1);
+        else e = -1;
+    }
+    __syncthreads();
+    int n = 0;
+    if (e >= 0 && r == 0) n = cnt[e];
+    __syncthreads();
+    if (n > 0) cnt[e] = atomicAdd(a.cnt + e, n);
+    __syncthreads();
+    if (on) {
+        const int64_t p = (int64_t)(blockIdx.x * PF_TKT + pt) * a.K + k;
+        a.ids[p] = e;
+        a.wts[p] = s_w[pt][k];
+        a.rank[p] = e >= 0 ? cnt[e] + r : 0;
+    }
 }
 
 // exclusive prefix sum of one int per thread over a 1024-thread group
@@ -176,96 +230,56 @@ __device__ __forceinline__ int excl_scan1024(int v, int* wsum, int* total) {
     return x - v + wsum[w];
 }
 
-// P3: one 1024-thread work-group.  Counting sort of the T*K pairs by expert
-// (the order of pairs inside an expert does not affect any result: every
-// pair's output row is computed on its own), the shared expert as expert E
-// with all T tokens, and the list of tiles of up to tile_pairs pairs.  Thread i owns experts
-// 2i and 2i+1 in the scans.
+// P3: counting sort of the T*K pairs by expert (the order of pairs inside an
+// expert does not affect any result: every pair's output row is computed on
+// its own), the shared expert as expert E with all T tokens, and the list of
+// tiles of up to tile_pairs pairs.  Every work-group scans the experts' counts
+// (thread i: experts 2i and 2i+1) and places its 1024 pairs; the first one
+// also writes the tiles.  (One work-group counting and placing all pairs:
+// 4096 tokens top-8 40 us.)
 __global__ __launch_bounds__(1024) void k_pf_plan(PfArgs a) {
-    __shared__ int cnt[2 * 1024], fill[MAX_E + 1];
+    __shared__ int first[2 * 1024];
     __shared__ int wsum[16], tot[2];
-    const int tid = threadIdx.x, TK = a.T * a.K, NE = a.E + 1;
-    for (int e = tid; e < 2 * 1024; e += 1024) cnt[e] = 0;
-    for (int e = tid; e < NE; e += 1024) fill[e] = 0;
-    for (int i = tid; i < a.tile_slots; i += 1024) a.tiles[i] = make_int4(0, 0, 0, 0);
-    __syncthreads();
-    // pairs in batches of 4 per thread: the 4 id loads (and weight loads)
-    // are issued together (one memory round trip per batch, not per pair);
-    // the first batch's ids and weights stay in registers for the scatter
-    int k4[4];
-    float kw[4];
-    for (int p0 = tid; p0 < TK; p0 += 4 * 1024) {
-        int e4[4];
-        float w4[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const bool in = p0 + i * 1024 < TK;
-            e4[i] = in ? a.ids[p0 + i * 1024] : -1;
-            w4[i] = in && a.ids_out ? a.wts[p0 + i * 1024] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (e4[i] >= 0) atomicAdd(&cnt[e4[i]], 1);
-        if (p0 == tid) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) { k4[i] = e4[i]; kw[i] = w4[i]; }
-        }
-    }
-    if (tid == 0) cnt[a.E] = a.has_shared ? a.T : 0;
-    __syncthreads();
-    const int c0 = cnt[2 * tid], c1 = cnt[2 * tid + 1];
-    const int TP = a.tile_pairs;
-    const int n0 = (c0 + TP - 1) / TP, n1 = (c1 + TP - 1) / TP;
+    const int tid = threadIdx.x, TK = a.T * a.K, E = a.E, TP = a.tile_pairs;
+    const int p = blockIdx.x * 1024 + tid, e = p < TK ? a.ids[p] : -1;
+    const int rank = p < TK ? a.rank[p] : 0;
+    if (blockIdx.x == 0)
+        for (int i = tid; i < a.tile_slots; i += 1024) a.tiles[i] = make_int4(0, 0, 0, 0);
+    const int c0 = 2 * tid < E ? a.cnt[2 * tid] : 0, c1 = 2 * tid + 1 < E ? a.cnt[2 * tid + 1] : 0;
     const int po = excl_scan1024(c0 + c1, wsum, &tot[0]);
-    const int to = excl_scan1024(n0 + n1, wsum, &tot[1]);
+    first[2 * tid] = po;
+    first[2 * tid + 1] = po + c0;
     __syncthreads();
-    cnt[2 * tid] = po;                 // cnt now holds each expert's first position
-    cnt[2 * tid + 1] = po + c0;
+    if (e >= 0) {
+        const int pos = first[e] + rank;
+        a.spairs[pos] = p;
+        a.stok[pos] = p / a.K;
+        if (a.ids_out) { a.ids_out[p] = e; a.w_out[p] = a.wts[p]; }
+    }
+    if (a.has_shared && p < a.T) {
+        a.spairs[tot[0] + p] = TK + p;
+        a.stok[tot[0] + p] = p;
+    }
+    if (blockIdx.x != 0) return;
     // tile -> slot 8 g + x of XCD x: the shared expert's tiles (full ones, and
     // of the slower types) come first, dealt one by one; then XCD x has a
     // contiguous eighth of the experts' tiles (those of one expert share its
-    // weights in that L2)
-    const int nsh = a.has_shared ? (a.T + TP - 1) / TP : 0, ne = tot[1] - nsh;
-    const int per = (ne + 7) >> 3, persh = (nsh + 7) >> 3;
+    // weights in that L2).  With the shared tiles last in one contiguous split
+    // one XCD had them all: 4096 tokens IQ3_S + Q5_K gate/up 774 against 562 us.
+    const int n0 = (c0 + TP - 1) / TP, n1 = (c1 + TP - 1) / TP;
+    const int to = excl_scan1024(n0 + n1, wsum, &tot[1]);
+    __syncthreads();
+    const int nsh = a.has_shared ? (a.T + TP - 1) / TP : 0, ne = tot[1];
+    const int per = max((ne + 7) >> 3, 1), persh = (nsh + 7) >> 3;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const int e = 2 * tid + h, c = h ? c1 : c0, base = h ? po + c0 : po, tb = h ? to + n0 : to;
+        const int c = h ? c1 : c0, base = h ? po + c0 : po, tb = h ? to + n0 : to;
         for (int s = 0; s * TP < c; s++) {
-            const int t = tb + s, x = t / max(per, 1);
-            const int slot = e == a.E ? s : 8 * (persh + t - x * per) + x;
-            a.tiles[slot] = make_int4(e, base + s * TP, min(TP, c - s * TP), 0);
+            const int t = tb + s, x = t / per;
+            a.tiles[8 * (persh + t - x * per) + x] = make_int4(2 * tid + h, base + s * TP, min(TP, c - s * TP), 0);
         }
     }
-    __syncthreads();
-    for (int p0 = tid; p0 < TK; p0 += 4 * 1024) {
-        int e4[4];
-        float w4[4];
-        if (p0 == tid) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) { e4[i] = k4[i]; w4[i] = kw[i]; }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const bool in = p0 + i * 1024 < TK;
-                e4[i] = in ? a.ids[p0 + i * 1024] : -1;
-                w4[i] = in && a.ids_out ? a.wts[p0 + i * 1024] : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int p = p0 + i * 1024, e = e4[i];
-            if (e < 0) continue;
-            const int pos = cnt[e] + atomicAdd(&fill[e], 1);
-            a.spairs[pos] = p;
-            a.stok[pos] = p / a.K;
-            if (a.ids_out) { a.ids_out[p] = e; a.w_out[p] = w4[i]; }
-        }
-    }
-    if (a.has_shared)
-        for (int t = tid; t < a.T; t += 1024) {
-            a.spairs[cnt[a.E] + t] = TK + t;
-            a.stok[cnt[a.E] + t] = t;
-        }
+    for (int s = tid; s < nsh; s += 1024) a.tiles[s] = make_int4(E, tot[0] + s * TP, min(TP, a.T - s * TP), 0);
 }
 
 // P6: grid (ceil(H/256), T): out = sum_k fmaf(w_k, dn_k, acc) (+ shared expert)
@@ -311,18 +325,23 @@ __global__ __launch_bounds__(256) void k_pf_combine(PfArgs a) {
 }
 
 struct PfPlan {
-    size_t logits, glogit, ids, wts, spairs, stok, tiles, dn, xh, xd, xs, hh, hd, hs, total;
+    size_t logits, glogit, ids, wts, cnt, rank, spairs, stok, tiles, dn, xh, xd, xs, hh, hd, hs, total;
     int tile_slots, tile_pairs;
 };
 
 static size_t al256p(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Pairs per GEMM tile, by the average pairs per expert: a weight block is
-// decoded once per tile, so tiles should hold an expert's pairs, but a wider
+// decoded once per tile, so a tile should hold an expert's pairs, but a wider
 // tile's LDS and registers leave two work-groups per CU instead of three.
+// H = 2048, F = 512, E = 256, top-8, 16 / 32 / 64 pairs: IQ3_S + Q5_K shared
+// 350 tokens (average 11) 186 / 202 / 217 us, 512 (16) 238 / 219 / 226, 800
+// (25) 321 / 271 / 265; Q4_0 350 173 / 185 / 196, 512 206 / 202 / 206, 800
+// 271 / 237 / 231; Q8_0 350 254 / 257 / 263, 512 297 / 274 / 276, 800 364 /
+// 306 / 305.
 static int pf_tile_pairs(int E, int K, int T) {
     const double avg = (double)T * K / E;
-    return avg <= 4 ? PF_PT : avg <= 24 ? 2 * PF_PT : 4 * PF_PT;
+    return avg <= 13 ? PF_PT : avg <= 20 ? 2 * PF_PT : 4 * PF_PT;
 }
 
 static PfPlan plan_pf(int H, int F, int E, int K, int T) {
@@ -339,6 +358,8 @@ static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     take(p.glogit, (size_t)T * 4);
     take(p.ids, (size_t)T * K * 4);
     take(p.wts, (size_t)T * K * 4);
+    take(p.cnt, (size_t)E * 4);
+    take(p.rank, (size_t)T * K * 4);
     take(p.spairs, P * 4);
     take(p.stok, P * 4);
     take(p.tiles, (size_t)slots(PF_PT) * sizeof(int4));
@@ -357,9 +378,9 @@ static void launch_pf(const PfArgs& a, int te, int ts, hipStream_t s) {
     hipLaunchKernelGGL(k_pf_router,
                        dim3(((a.E + (a.sh_gate_w ? 1 : 0) + PF_RE - 1) / PF_RE) * ((a.T + PF_RT - 1) / PF_RT)),
                        dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_pf_quant, dim3(a.H / QK / 8, a.T), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_pf_topk, dim3(a.T), dim3(64), 0, s, a);
-    hipLaunchKernelGGL(k_pf_plan, dim3(1), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(k_pf_quant, dim3((unsigned)(((int64_t)a.T * (a.H / QK) + 31) / 32)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_pf_topk, dim3((a.T + PF_TKT - 1) / PF_TKT), dim3(64 * PF_TKT), 0, s, a);
+    hipLaunchKernelGGL(k_pf_plan, dim3((a.T * a.K + 1023) / 1024), dim3(1024), 0, s, a);
     if (te == T_Q4_0) pf_launch_experts<T_Q4_0>(a, ts, s);
     else if (te == T_Q8_0) pf_launch_experts<T_Q8_0>(a, ts, s);
     else pf_launch_experts<T_IQ3_S>(a, ts, s);
@@ -419,6 +440,7 @@ void chimere_moe_prefill(const chimere_moe_layer* L, const float* x, float* out,
     a.ids_out = ids_out; a.w_out = w_out;
     a.logits = (float*)(w + p.logits); a.glogit = (float*)(w + p.glogit);
     a.ids = (int*)(w + p.ids); a.wts = (float*)(w + p.wts);
+    a.cnt = (int*)(w + p.cnt); a.rank = (int*)(w + p.rank);
     a.spairs = (int*)(w + p.spairs);
     a.stok = (int*)(w + p.stok); a.tiles = (int4*)(w + p.tiles);
     a.dn = (float*)(w + p.dn);
