@@ -95,6 +95,142 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq(MmvqArgs a) {
     }
 }
 
+// Several tokens: the block dots on v_mfma_i32_4x4x4_16b_i8, whose 16
+// independent 4x4 products are the 16 slots of the fp32 order: lane 4 j + i
+// decodes block j (mod 16) of row i of its wave's four rows and is the B column
+// of token 4 n + i, so a wave makes the exact int32 dots of 4 rows x 4 tokens x
+// 16 blocks in eight instructions, and acc[n][r] of lane 4 j + i is slot j of
+// (row r, token 4 n + i).  With the dots as eight v_dot4 per (block, token),
+// every lane read every token's block from LDS: 151936x2048 Q6_K, 8 tokens, was
+// bound by those reads (320 bytes per lane and block) and its vector ALU (about
+// 200 instructions per lane and block): 106 -> 83 us.  The tokens' blocks stay
+// raw in LDS: decoded there by every work-group (512 blocks for its 16 rows) the
+// same case took 89 us, Q4_0 78 us against 58.
+// LDS bytes between tokens' rows of a chunk (raw Q8_1 blocks, copied
+// asynchronously): 16 more than the blocks', so that the four tokens a lane
+// quad reads are on different banks
+constexpr int XTOK_ROW = MMVQ_BLOCKS * Q8_1_BYTES + 16;
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// value of lane 4 j + R of the quad
+template <int R>
+__device__ __forceinline__ float quad_of(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x55 * R, 0xF, 0xF, true));
+}
+
+template <int T, int NG>
+__global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_tok(MmvqArgs a) {
+    constexpr int CBLK = MMVQ_BLOCKS, CB = chunk_bytes<T>(CBLK), PAD = mmvq_pad<T>();
+    __shared__ __attribute__((aligned(16))) uint8_t tile[TILE_ROWS * (CB + PAD) + 16];
+    __shared__ __attribute__((aligned(16))) uint8_t xs[4 * NG * XTOK_ROW];
+    __shared__ uint32_t grid[T == T_IQ3_S ? 512 : 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane >> 2, i = lane & 3;
+    const int r0 = blockIdx.x * TILE_ROWS, nr = min(TILE_ROWS, a.nrows - r0);
+    const int64_t rb = row_bytes(T, a.ncols);
+    const uint8_t* W = a.W + (int64_t)r0 * rb;
+    const int nb = a.ncols / QK;
+    if constexpr (T == T_IQ3_S)
+        for (int k = tid; k < 512; k += GEMV_THREADS) grid[k] = c_iq3s_grid_mmvq[k];
+    float acc[NG][4];
+#pragma unroll
+    for (int n = 0; n < NG; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[n][r] = 0.0f;
+    for (int b0 = 0; b0 < nb; b0 += CBLK) {
+        const int cb = min(CBLK, nb - b0), seg = chunk_bytes<T>(cb);
+        const int64_t goff = (int64_t)b0 / (QTraits<T>::ELEMS / QK) * QTraits<T>::BYTES;
+        const bool al16 = (((uintptr_t)W | (uintptr_t)rb | (uintptr_t)goff | (uintptr_t)seg) & 15) == 0;
+        const bool xal = (((uintptr_t)a.x | (uintptr_t)a.x_tok_stride | (uintptr_t)(cb * Q8_1_BYTES)) & 15) == 0;
+        const int lseg = PAD && al16 ? seg + PAD : seg;
+        __syncthreads();   // every wave is done with the previous chunk
+        bool staged = false;
+        if constexpr (CB % 16 == 0)
+            if (al16 && cb == CBLK) {
+                stage_rows_fixed<CB, CB + PAD, 16, TILE_ROWS, GEMV_THREADS, CPOL_STREAM, true>(tile, W + goff, nr, nullptr,
+                                                                                             rb, nr, tid);
+                staged = true;
+            }
+        if (!staged) stage_rows<stage_dw<T>(), CPOL_STREAM>(tile, W + goff, rb, nr, seg, tid, GEMV_THREADS, lseg);
+        // tokens past the last repeat it (their sums are not stored); a
+        // wave copies whole tokens
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const int t = 4 * k + wave;
+            const uint8_t* src = a.x + min(t, a.ntok - 1) * a.x_tok_stride + (int64_t)b0 * Q8_1_BYTES;
+            if (xal)
+                for (int c = 0; c < cb * Q8_1_BYTES / 16; c += 64) {
+                    if (c + lane < cb * Q8_1_BYTES / 16)
+                        __builtin_amdgcn_global_load_lds((const glb_void_t*)(src + (c + lane) * 16),
+                                                         (lds_void_t*)(xs + t * XTOK_ROW + c * 16), 16, 0, 0);
+                }
+            else
+                for (int c = 0; c < cb * Q8_1_BYTES / 4; c += 64)
+                    if (c + lane < cb * Q8_1_BYTES / 4)
+                        __builtin_amdgcn_global_load_lds((const glb_void_t*)(src + (c + lane) * 4),
+                                                         (lds_void_t*)(xs + t * XTOK_ROW + c * 4), 4, 0, 0);
+        }
+        lds_copy_wait();
+        __syncthreads();
+        const uint8_t* row = tile + min(4 * wave + i, nr - 1) * lseg;   // rows past the last repeat it
+#pragma unroll 1
+        for (int bg = 0; bg < cb; bg += SLOTS) {
+            const bool in = bg + j < cb;
+            const int b = in ? bg + j : cb - 1;
+            WBlk w;
+            block_decode<T>(row, b, grid, w);
+            const float mu = T == T_IQ3_S || T == T_Q4_K || T == T_Q5_K || T == T_Q6_K ? (float)w.mult : 0.0f;
+            const float mu2 = T == T_Q6_K ? (float)w.mult2 : 0.0f, mm = (float)w.mmin;
+#pragma unroll
+            for (int n = 0; n < NG; n++) {
+                XBlk x;   // token 4 n + i's block; sums where the type needs them
+                const uint32_t* xw = (const uint32_t*)(xs + (4 * n + i) * XTOK_ROW + b * Q8_1_BYTES);
+                x.d = h2f(xw[0] & 0xFFFFu);
+                int lo = 0, sq = 0;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    x.q[e] = (int)xw[1 + e];
+                    if (needs_sumq<T>()) (T == T_Q6_K && e < 4 ? lo : sq) = dot4(x.q[e], 0x01010101, T == T_Q6_K && e < 4 ? lo : sq);
+                }
+                // Q4_0: -8 sum q; Q6_K: -32 sum q of each half
+                const int c0 = T == T_Q4_0 ? -8 * sq : T == T_Q6_K ? -32 * lo : 0, c1 = T == T_Q6_K ? -32 * sq : 0;
+                v4i s = {c0, c0, c0, c0}, s2 = {c1, c1, c1, c1};
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    if (T == T_Q6_K && e >= 4) s2 = __builtin_amdgcn_mfma_i32_4x4x4i8(w.v[e], x.q[e], s2, 0, 0, 0);
+                    else s = __builtin_amdgcn_mfma_i32_4x4x4i8(w.v[e], x.q[e], s, 0, 0, 0);
+                }
+                auto row_acc = [&](auto rtag) {
+                    constexpr int R = decltype(rtag)::value;
+                    // the exact block dot: its factors are integers below 2^24
+                    float v = (float)s[R];
+                    if constexpr (T == T_Q6_K) v = __builtin_fmaf((float)s2[R], quad_of<R>(mu2), v * quad_of<R>(mu));
+                    else if constexpr (T == T_IQ3_S || T == T_Q4_K || T == T_Q5_K) v = v * quad_of<R>(mu);
+                    float o = __builtin_fmaf(quad_of<R>(w.dw) * x.d, v, acc[n][R]);
+                    if constexpr (T == T_Q4_K || T == T_Q5_K)
+                        o = __builtin_fmaf(-(quad_of<R>(w.dm) * x.d), quad_of<R>(mm) * (float)sq, o);
+                    acc[n][R] = in ? o : acc[n][R];
+                };
+                row_acc(std::integral_constant<int, 0>{});
+                row_acc(std::integral_constant<int, 1>{});
+                row_acc(std::integral_constant<int, 2>{});
+                row_acc(std::integral_constant<int, 3>{});
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NG; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            // the halving tree over the slots: xor 8, 4, 2, 1 of j
+            float v = acc[n][r];
+            v = v + xlane<32>(v);
+            v = v + xlane<16>(v);
+            v = v + xlane<8>(v);
+            v = v + xlane<4>(v);
+            if (j == 0 && 4 * n + i < a.ntok && 4 * wave + r < nr) a.y[(4 * n + i) * a.y_tok_stride + r0 + 4 * wave + r] = v;
+        }
+}
+
 // One token, rows of exactly NCH 64-block chunks (2048 * NCH columns), whole
 // 16-row tiles, 16-byte aligned rows: the tile's copies, the activation
 // blocks, the dots and the L=16 tree with compile-time sizes and a
@@ -168,10 +304,30 @@ static void launch_t(const MmvqArgs& a, int nslots, hipStream_t s) {
         hipLaunchKernelGGL((k_mmvq<T, 1, true>), grid, blk, 0, s, a);
         return;
     }
-    switch (a.ntok) {
-#define CASE(N) case N: hipLaunchKernelGGL((k_mmvq<T, N>), grid, blk, 0, s, a); break;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
-#undef CASE
+    if constexpr (T == T_Q4_0S) {   // one token only
+        hipLaunchKernelGGL((k_mmvq<T, 1>), grid, blk, 0, s, a);
+    } else {
+        // k_mmvq_tok works for four tokens at a time: measured (us, k_mmvq /
+        // k_mmvq_tok, 151936x2048) 2 tokens Q4_0 30.8 / 39.5, Q6_K 54 / 57; 3
+        // tokens Q5_K 47.3 / 48.5; 4 tokens Q4_0 42.7 / 36.7, Q6_K 66 / 55; 5
+        // tokens Q4_0 53 / 57, Q5_K 60 / 77; 8 tokens Q8_0 133 / 84, Q4_0 69 /
+        // 58, Q5_K 85 / 77, Q6_K 106 / 83, IQ3_S 80 / 64, MXFP4 74 / 61; the
+        // K-quants with a min term break even at seven
+        constexpr bool KQ = T == T_Q4_K || T == T_Q5_K;
+        switch (a.ntok) {
+        case 1: hipLaunchKernelGGL((k_mmvq<T, 1>), grid, blk, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((k_mmvq<T, 2>), grid, blk, 0, s, a); break;
+        case 3: hipLaunchKernelGGL((k_mmvq<T, 3>), grid, blk, 0, s, a); break;
+        case 4: hipLaunchKernelGGL((k_mmvq_tok<T, 1>), grid, blk, 0, s, a); break;
+        case 5: hipLaunchKernelGGL((k_mmvq<T, 5>), grid, blk, 0, s, a); break;
+        case 6:
+            if constexpr (KQ) {
+                hipLaunchKernelGGL((k_mmvq<T, 6>), grid, blk, 0, s, a);
+                break;
+            }
+            [[fallthrough]];
+        default: hipLaunchKernelGGL((k_mmvq_tok<T, 2>), grid, blk, 0, s, a); break;
+        }
     }
 }
 

@@ -304,3 +304,28 @@ def test_f32_gemv_is_quantizer_plus_gemv(dev, t, nrows, ncols):
         fn(w, xd, y, scratch, nrows, ncols)
         assert (host(scratch) == host(xq).reshape(-1)).all()
         assert (host(y).view(np.uint32) == host(want).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("t", [O.Q8_0, O.Q4_0, O.IQ3_S, O.Q4_K, O.Q5_K, O.Q6_K, O.MXFP4])
+@pytest.mark.parametrize("nrows,ncols,ntok,off", [
+    (16, 256, 4, 0), (35, 2048, 4, 0), (50, 2304, 8, 0),      # fewer than 16 blocks; short tiles; a ragged chunk
+    (33, 4096, 6, 0), (64, 2048, 7, 0), (20, 1280, 8, 4),     # short token groups; inputs only 4-byte aligned
+])
+def test_multi_token_on_matrix_cores(dev, t, nrows, ncols, ntok, off):
+    """Four and six to eight tokens (the 16-slot matrix products): bit-exact
+    against the oracle's (L=16, G=1) order."""
+    print(f"multi type={t} {nrows}x{ncols} ntok={ntok} off={off}", flush=True)
+    rng = np.random.default_rng(nrows + ncols + ntok + t)
+    if t in (O.Q8_0, O.Q4_0, O.IQ3_S):
+        w = O.quantize(t, rng.normal(0, 0.02, (nrows, ncols)).astype(np.float32))
+    else:
+        w = npref.rand_kq(t, nrows, ncols, rng)
+    x = rng.standard_normal((ntok, ncols)).astype(np.float32)
+    x[0, :32] = 0
+    xq = O.quantize_q8_1(x)
+    buf = torch.zeros(xq.size + 16, dtype=torch.uint8, device=dev)
+    buf[off:off + xq.size] = dev_t(xq, dev).reshape(-1)
+    y = torch.zeros(ntok, nrows, dtype=torch.float32, device=dev)
+    G.gemv_multi(t, dev_t(w, dev), buf[off:], y, nrows, ncols, ntok)
+    yo = O.gemv(t, w, xq, ncols, nrows, ntok=ntok, xq_stride=xq.shape[1])
+    assert (host(y).view(np.uint32) == np.asarray(yo).reshape(ntok, nrows).view(np.uint32)).all()
