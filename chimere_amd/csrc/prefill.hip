@@ -121,13 +121,10 @@ __global__ __launch_bounds__(256) void k_pf_router(PfArgs a) {
     }
 }
 
-// Q8_1 of x (the values of k_quantize_q8_1) in the GEMMs' layout, and the
-// expert counts zeroed for k_pf_topk.  Eight lanes per block, 16-byte loads
+// Q8_1 of x (the values of k_quantize_q8_1) in the GEMMs' layout.  Eight lanes per block, 16-byte loads
 // (two half-waves per block with 4-byte loads and 2-byte stores: 4096 tokens
 // 19.7 us).  Grid: groups of 32 blocks of all tokens
 __global__ __launch_bounds__(256) void k_pf_quant(PfArgs a) {
-    if (blockIdx.x == 0)
-        for (int e = threadIdx.x; e < a.E; e += 256) a.cnt[e] = 0;
     const int64_t b = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
     const int i = threadIdx.x & 7;
     if (b >= (int64_t)a.T * (a.H / QK)) return;   // whole groups of eight lanes exit together
@@ -166,9 +163,10 @@ __global__ __launch_bounds__(256) void k_pf_quant(PfArgs a) {
     }
 }
 
-// P2: one wave per token, 16 tokens per work-group; the work-group's pairs are
-// counted per expert in LDS, and one global count per (work-group, expert)
-// gives each pair its rank among its expert's
+// P2: one wave per token, 16 tokens per work-group; each pair's rank among the
+// work-group's pairs of its expert, and the work-group's count of every expert
+// (counted in global memory instead, the returning atomics of 4096 tokens took
+// 15 us)
 constexpr int PF_TKT = 16;
 __global__ __launch_bounds__(64 * PF_TKT) void k_pf_topk(PfArgs a) {
     __shared__ uint64_t s_tk[PF_TKT][128];
@@ -187,18 +185,14 @@ __global__ __launch_bounds__(64 * PF_TKT) void k_pf_topk(PfArgs a) {
         if ((unsigned)e < (unsigned)a.E) r = atomicAdd(&cnt[e], 1);
         else e = -1;
     }
-    __syncthreads();
-    int n = 0;
-    if (e >= 0 && r == 0) n = cnt[e];
-    __syncthreads();
-    if (n > 0) cnt[e] = atomicAdd(a.cnt + e, n);
-    __syncthreads();
     if (on) {
         const int64_t p = (int64_t)(blockIdx.x * PF_TKT + pt) * a.K + k;
         a.ids[p] = e;
         a.wts[p] = s_w[pt][k];
-        a.rank[p] = e >= 0 ? cnt[e] + r : 0;
+        a.rank[p] = r;
     }
+    __syncthreads();
+    for (int i = tid; i < a.E; i += 64 * PF_TKT) a.cnt[(int64_t)blockIdx.x * a.E + i] = cnt[i];
 }
 
 // exclusive prefix sum of one int per thread over a 1024-thread group
@@ -231,34 +225,64 @@ __device__ __forceinline__ int excl_scan1024(int v, int* wsum, int* total) {
 }
 
 // P3: counting sort of the T*K pairs by expert (the order of pairs inside an
-// expert does not affect any result: every pair's output row is computed on
-// its own), the shared expert as expert E with all T tokens, and the list of
-// tiles of up to tile_pairs pairs.  Every work-group scans the experts' counts
-// (thread i: experts 2i and 2i+1) and places its 1024 pairs; the first one
-// also writes the tiles.  (One work-group counting and placing all pairs:
-// 4096 tokens top-8 40 us.)
+// expert -- by token here -- does not affect any result: every pair's output
+// row is computed on its own), the shared expert as expert E with all T
+// tokens, and the list of tiles of up to tile_pairs pairs.  Every work-group
+// sums the counts of all top-k work-groups (each expert's total, and what comes
+// before its own PF_PLG of them), scans the totals (thread i: experts 2i and
+// 2i+1) and places its pairs; the first one also writes the tiles.  (One
+// work-group counting and placing all pairs: 4096 tokens top-8 40 us.)
+constexpr int PF_PLG = 4;   // top-k work-groups (64 tokens, at most 1024 pairs) per plan work-group
 __global__ __launch_bounds__(1024) void k_pf_plan(PfArgs a) {
-    __shared__ int first[2 * 1024];
+    __shared__ int first[1024], total[1024], before[1024];
     __shared__ int wsum[16], tot[2];
     const int tid = threadIdx.x, TK = a.T * a.K, E = a.E, TP = a.tile_pairs;
-    const int p = blockIdx.x * 1024 + tid, e = p < TK ? a.ids[p] : -1;
-    const int rank = p < TK ? a.rank[p] : 0;
+    const int ntk = (a.T + PF_TKT - 1) / PF_TKT, g0 = blockIdx.x * PF_PLG;
+    const int p0 = blockIdx.x * PF_PLG * PF_TKT * a.K, np = min(TK - p0, PF_PLG * PF_TKT * a.K);
+    const int e = tid < np ? a.ids[p0 + tid] : -1;
+    const int rank = tid < np ? a.rank[p0 + tid] : 0;
     if (blockIdx.x == 0)
         for (int i = tid; i < a.tile_slots; i += 1024) a.tiles[i] = make_int4(0, 0, 0, 0);
-    const int c0 = 2 * tid < E ? a.cnt[2 * tid] : 0, c1 = 2 * tid + 1 < E ? a.cnt[2 * tid + 1] : 0;
+    total[tid] = 0;
+    before[tid] = 0;
+    __syncthreads();
+    {
+        // 1024 / EP threads per expert, each over every (1024 / EP)-th top-k work-group
+        const int EP = E <= 256 ? 256 : E <= 512 ? 512 : 1024, seg = tid / EP, nseg = 1024 / EP, ex = tid - seg * EP;
+        if (ex < E) {
+            int s = 0, sb = 0;
+#pragma unroll 8
+            for (int g = seg; g < ntk; g += nseg) {
+                const int c = a.cnt[(int64_t)g * E + ex];
+                s += c;
+                sb += g < g0 ? c : 0;
+            }
+            atomicAdd(&total[ex], s);
+            atomicAdd(&before[ex], sb);
+        }
+    }
+    __syncthreads();
+    const int c0 = tid < 512 ? total[2 * tid] : 0, c1 = tid < 512 ? total[2 * tid + 1] : 0;
     const int po = excl_scan1024(c0 + c1, wsum, &tot[0]);
-    first[2 * tid] = po;
-    first[2 * tid + 1] = po + c0;
+    if (tid < 512) {
+        first[2 * tid] = po;
+        first[2 * tid + 1] = po + c0;
+    }
     __syncthreads();
     if (e >= 0) {
-        const int pos = first[e] + rank;
+        // the pair's top-k work-group is g0 + tid / (16 K): the counts of the
+        // plan work-group's earlier ones come before it too
+        int pos = first[e] + before[e] + rank;
+        for (int g = g0; g < g0 + tid / (PF_TKT * a.K); g++) pos += a.cnt[(int64_t)g * E + e];
+        const int p = p0 + tid;
         a.spairs[pos] = p;
         a.stok[pos] = p / a.K;
         if (a.ids_out) { a.ids_out[p] = e; a.w_out[p] = a.wts[p]; }
     }
-    if (a.has_shared && p < a.T) {
-        a.spairs[tot[0] + p] = TK + p;
-        a.stok[tot[0] + p] = p;
+    const int t0 = blockIdx.x * PF_PLG * PF_TKT;
+    if (a.has_shared && tid < PF_PLG * PF_TKT && t0 + tid < a.T) {
+        a.spairs[tot[0] + t0 + tid] = TK + t0 + tid;
+        a.stok[tot[0] + t0 + tid] = t0 + tid;
     }
     if (blockIdx.x != 0) return;
     // tile -> slot 8 g + x of XCD x: the shared expert's tiles (full ones, and
@@ -358,7 +382,7 @@ static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     take(p.glogit, (size_t)T * 4);
     take(p.ids, (size_t)T * K * 4);
     take(p.wts, (size_t)T * K * 4);
-    take(p.cnt, (size_t)E * 4);
+    take(p.cnt, (size_t)((T + PF_TKT - 1) / PF_TKT) * E * 4);
     take(p.rank, (size_t)T * K * 4);
     take(p.spairs, P * 4);
     take(p.stok, P * 4);
@@ -380,7 +404,7 @@ static void launch_pf(const PfArgs& a, int te, int ts, hipStream_t s) {
                        dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_pf_quant, dim3((unsigned)(((int64_t)a.T * (a.H / QK) + 31) / 32)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_pf_topk, dim3((a.T + PF_TKT - 1) / PF_TKT), dim3(64 * PF_TKT), 0, s, a);
-    hipLaunchKernelGGL(k_pf_plan, dim3((a.T * a.K + 1023) / 1024), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(k_pf_plan, dim3((a.T + PF_PLG * PF_TKT - 1) / (PF_PLG * PF_TKT)), dim3(1024), 0, s, a);
     if (te == T_Q4_0) pf_launch_experts<T_Q4_0>(a, ts, s);
     else if (te == T_Q8_0) pf_launch_experts<T_Q8_0>(a, ts, s);
     else pf_launch_experts<T_IQ3_S>(a, ts, s);

@@ -50,8 +50,8 @@ struct PfArgs {
     float* glogit;   // [T]
     int* ids;        // [T*K]
     float* wts;      // [T*K]
-    int* cnt;        // [E] pairs of each expert
-    int* rank;       // [T*K] a pair's place among its expert's
+    int* cnt;        // [top-k work-groups][E] pairs of each expert
+    int* rank;       // [T*K] a pair's place among its expert's of its top-k work-group
     int* spairs;     // [T*K + T] pairs grouped by expert (shared expert last)
     int* stok;       // [T*K + T] the pairs' tokens, in the same order
     int4* tiles;     // [tile_slots] (expert, first position in spairs, pairs or 0)
