@@ -158,8 +158,9 @@ __global__ __launch_bounds__(256) void k_pf_quant(PfArgs a) {
     sq += xlane<1>(sq);
     *(v4h*)(a.xh + b * QK + 4 * i) = h;
     if (i == 0) {
-        a.xd[b] = f2h(d);
-        a.xs[b] = (float)sq;
+        const uint32_t dh = f2h(d);
+        a.xd[b] = dh;
+        a.xs[b] = h2f(dh) * (float)sq;   // exact: 11 x 12 bits
     }
 }
 

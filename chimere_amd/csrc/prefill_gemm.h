@@ -58,7 +58,8 @@ struct PfArgs {
     float* dn;       // [T*K + T][H] down-projection output per pair
     // Q8_1 blocks of x (by token) and of h (by position in spairs) as the
     // GEMMs read them: the quants as f16, the block's f16 scale in the low
-    // half of a word, the sum of its quants
+    // half of a word, and (for the K-quants' min terms) that scale times the sum of
+    // its quants, exact in f32
     _Float16 *xh, *hh;
     uint32_t *xd, *hd;
     float *xs, *hs;
@@ -291,7 +292,7 @@ template <> struct PfRow<T_Q6_K> {
 
 // ---- LDS of one work-group: two stages of the weight rows' chunks, of the
 // activation blocks (units of 8 pairs x 2 blocks) and of their scales
-// ([pair][block]; K-quants also the quant sums)
+// ([pair][block]; K-quants also d_x * sum q_x)
 struct PfLds {
     uint8_t* smem;
     uint32_t* sd;
@@ -381,7 +382,7 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
         xp[j] = (const uint8_t*)(xh + (int64_t)rowof(8 * grp + r) * (nb * 32)) + (MT > 1 ? 0 : 128 * NXB * (wave >> 1)) +
                 16 * ((lane & 7) ^ r);
     }
-    // scales (wave 0), K-quants' quant sums (wave 1): a pair's 4 blocks per lane
+    // scales (wave 0), K-quants' d_x * sum q_x (wave 1): a pair's 4 blocks per lane
     const uint32_t* dp = (wave ? (const uint32_t*)xs : xd) + (lane < 16 * MT ? (int64_t)rowof(lane) * nb : 0);
 
     auto issue_x = [&](int st, int p) {   // activation stage st of the row, into stage p
@@ -443,7 +444,7 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
             v4f s0[NG][MT], s1[NG][MT];
             v16f t[NG];
             uint32_t dx[CH], dwv[NG];
-            float m0[NG], m1[NG], kd[CH][MT][4], ks[CH][MT][4];   // K-quants: scales and quant sums of the lane's outputs
+            float m0[NG], m1[NG], ks[CH][MT][4];   // Q6_K half scales; K-quants: d_x * sum q_x of the lane's outputs
             const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
             const v16f z16 = {0.0f};
             auto do_load = [&](int g) {
@@ -465,9 +466,7 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
                     for (int m = 0; m < MT; m++)
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
-                            const int e = (16 * m + 4 * q + i) * 4 + dq;
-                            kd[b][m][i] = h2f(L.d(st & 1)[e]);
-                            ks[b][m][i] = L.s(st & 1)[e];
+                            ks[b][m][i] = L.s(st & 1)[(16 * m + 4 * q + i) * 4 + dq];
                         }
                 }
             };
@@ -499,9 +498,9 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
                         // Q6_K: lo * sc0 + hi * sc1, both products and the sum exact
                         const float sv = T == T_Q6_K ? __builtin_fmaf(s1[g][m][i], m1[g], s0[g][m][i] * m0[g]) : s0[g][m][i];
                         float o = __builtin_fmaf(t[tg][ti], sv, acc[n][m][i]);
-                        // the K-quants' min term: fmaf(-(f32(dmin) * f32(d_x)), (float)(m * sum q_x), acc)
-                        if constexpr (pf_kq<T>())
-                            o = __builtin_fmaf(row[n].neg_dmin() * kd[b][m][i], row[n].min_of(b) * ks[b][m][i], o);
+                        // the K-quants' min term fmaf(-(f32(dmin) * f32(d_x)), (float)(m * sum q_x),
+                        // acc), its exact product as -(dmin * m) times d_x * sum q_x (both exact)
+                        if constexpr (pf_kq<T>()) o = __builtin_fmaf(row[n].neg_dmin() * row[n].min_of(b), ks[b][m][i], o);
                         asm volatile("" : "+v"(o));   // the rescale stays in its group (it would sink below the products)
                         acc[n][m][i] = o;
                     }
@@ -588,12 +587,13 @@ __device__ __forceinline__ int4 pf_place(const PfArgs& a, int nslice, int& sl) {
         copy16_lds_untracked((const uint4*)c_iq3s_hgrid.w + threadIdx.x, (uint4*)grid + (threadIdx.x & ~63u))
 
 // The tile's pairs against type T: run(type, pair tiles, first position, pairs)
-template <int TE, int TS, int MT, class Run>
+template <int TE, int TS, int MT, int MKQ, class Run>
 __device__ __forceinline__ void pf_dispatch(const int4& ti, bool sh, Run run) {
     auto with = [&](auto ttag) {
-        // the K-quants' min terms and Q6_K's second products leave registers
-        // for 32 pairs at a time
-        constexpr int T = decltype(ttag)::value, M = (pf_kq<T>() || T == T_Q6_K) && MT > 2 ? 2 : MT;
+        // Q6_K's second products leave registers for 32 pairs at a time, the
+        // K-quants' min terms for 16 * MKQ
+        constexpr int T = decltype(ttag)::value, MX = T == T_Q6_K ? 2 : pf_kq<T>() ? MKQ : 4,
+                      M = MT < MX ? MT : MX;
         if constexpr (M < MT) {
             for (int p = 0; p < ti.z; p += PF_PT * M) {
                 run(ttag, std::integral_constant<int, M>{}, ti.y + p, min(ti.z - p, PF_PT * M));
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void k_pf_gate_up(PfArgs a) {
     const uint8_t* g = sh ? a.sh_gate : a.gate + (int64_t)e * a.sg;
     const uint8_t* u = sh ? a.sh_up : a.up + (int64_t)e * a.su;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c = lane & 15;
-    pf_dispatch<TE, TS, MT>(ti, sh, [&](auto ttag, auto mtag, int start, int np) {
+    pf_dispatch<TE, TS, MT, 4>(ti, sh, [&](auto ttag, auto mtag, int start, int np) {
         constexpr int T = decltype(ttag)::value, M = decltype(mtag)::value;
         const int64_t rb = row_bytes(T, a.H);
         pf_gemm<T, M, pf_wdb<T, TE, TS>()>(L, g + f0 * rb, u + f0 * rb, rb, 1, 64 * rb, a.H / QK, a.xh, a.xd,
@@ -664,6 +664,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void k_pf_gate_up(PfArgs a) {
                     // (int8_t): where d underflows to 0 the byte the Q8_1 block would hold
                     const int qv = amax == 0.0f ? 0 : (int8_t)(int)__builtin_roundf(acc[0][m][i] / d);
                     acc[1][m][i] = (float)qv;
+                    am[m][i] = h2f(f2h(d));
                     if (p < np) {
                         a.hh[(int64_t)(start + p) * a.F + f0 + 16 * wave + c] = (_Float16)qv;
                         if (c == 0 && (wave & 1) == 0) a.hd[(start + p) * nb + (f0 >> 5) + (wave >> 1)] = f2h(d);
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void k_pf_gate_up(PfArgs a) {
                     for (int i = 0; i < 4; i++) {
                         const int p = 16 * m + 4 * q + i;
                         if (c == 0 && (wave & 1) == 0 && p < np)
-                            a.hs[(start + p) * nb + (f0 >> 5) + (wave >> 1)] = acc[1][m][i] + ex[(wave ^ 1) * 16 * M + p];
+                            a.hs[(start + p) * nb + (f0 >> 5) + (wave >> 1)] = am[m][i] * (acc[1][m][i] + ex[(wave ^ 1) * 16 * M + p]);
                     }
             }
         });
@@ -710,7 +711,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void k_pf_down(PfArgs a) {
     const bool sh = e == a.E;
     const uint8_t* d = sh ? a.sh_down : a.down + (int64_t)e * a.sd;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c = lane & 15;
-    pf_dispatch<TE, TS, MT>(ti, sh, [&](auto ttag, auto mtag, int start, int np) {
+    pf_dispatch<TE, TS, MT, 2>(ti, sh, [&](auto ttag, auto mtag, int start, int np) {
         constexpr int T = decltype(ttag)::value, M = decltype(mtag)::value;
         const int64_t rb = row_bytes(T, a.F);
         int prs[M][4];   // read here: a load between the slices would wait for the copies in flight
