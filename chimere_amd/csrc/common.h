@@ -487,17 +487,18 @@ __device__ __forceinline__ void wdec_mxfp4(const uint8_t* row, int off, WBlk& w)
 
 // Block b of a row chunk in LDS (layout as block_dot below), decoded.  SG:
 // IQ3_S lookups in the sign-folded codebook (Iq3sSignedGrid) instead of the
-// 512-word one.
+// 512-word one.  pre: bytes from `row` (4-byte aligned) to the chunk's start
+// (Q4_K / Q5_K: 0; even except for MXFP4).
 template <int T, bool SG = false>
-__device__ __forceinline__ void block_decode(const uint8_t* row, int b, const uint32_t* grid, WBlk& w) {
+__device__ __forceinline__ void block_decode(const uint8_t* row, int b, const uint32_t* grid, WBlk& w, int pre = 0) {
     if constexpr (T == T_Q8_0) {
-        const int off = b * 34;
+        const int off = pre + b * 34;
         uint32_t q[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) q[i] = lds_u32(row, off + 2 + 4 * i);
         wdec_q8_0_core(lds_u16(row, off), q, w);
     } else if constexpr (T == T_Q4_0 || T == T_Q4_0S) {
-        const int off = b * 18;
+        const int off = pre + b * 18;
         uint32_t qs[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) qs[i] = lds_u32(row, off + 2 + 4 * i);
@@ -507,11 +508,11 @@ __device__ __forceinline__ void block_decode(const uint8_t* row, int b, const ui
     } else if constexpr (T == T_Q5_K) {
         wdec_q5_k(row + (b >> 3) * 176, b & 7, w);
     } else if constexpr (T == T_Q6_K) {
-        wdec_q6_k(row, (b >> 3) * 210, b & 7, w);
+        wdec_q6_k(row, pre + (b >> 3) * 210, b & 7, w);
     } else if constexpr (T == T_MXFP4) {
-        wdec_mxfp4(row, b * 17, w);
+        wdec_mxfp4(row, pre + b * 17, w);
     } else {
-        const int off = (b >> 3) * 110, ib = b & 7;
+        const int off = pre + (b >> 3) * 110, ib = b & 7;
         const uint32_t sc = row[off + 106 + (ib >> 1)];
         wdec_iq3_s_core<SG>(lds_u16(row, off), lds_u32(row, off + 2 + 8 * ib), lds_u32(row, off + 6 + 8 * ib),
                         row[off + 66 + ib], lds_u32(row, off + 74 + 4 * ib), (sc >> (4 * (ib & 1))) & 0xFu, grid, w);
@@ -678,6 +679,27 @@ __device__ __forceinline__ void stage_rows_fixed(uint8_t* __restrict__ lds, cons
             else
                 __builtin_amdgcn_global_load_lds((const glb_void_t*)src, (lds_void_t*)(lds + c0 * 4), 4, 0, CPOL);
         }
+    }
+}
+
+// nrows row segments of `seg` bytes at g + r * gstride, any alignment, each as
+// the 16-byte aligned span holding it, to LDS rows of span_stride(seg) bytes:
+// row r's bytes start ((uintptr_t)(g + r * gstride) & 15) into its LDS row.
+// Reads only 16-byte granules that hold bytes of a segment (never outside a
+// mapped page).
+__device__ __forceinline__ int span_stride(int seg) { return (seg + 30) & ~15; }
+template <int CPOL>
+__device__ __forceinline__ void stage_row_spans(uint8_t* __restrict__ lds, const uint8_t* g, int64_t gstride, int nrows,
+                                                int seg, int tid, int nthreads) {
+    const int per = span_stride(seg) >> 4, tot = per * nrows;
+    const int lane = tid & 63, wave = tid >> 6, nw = nthreads >> 6;
+    for (int c0 = wave * 64; c0 < tot; c0 += nw * 64) {
+        const int c = c0 + lane, r = c / per, col = c - r * per;
+        const uint8_t* p = g + r * gstride;
+        const int pre = (int)((uintptr_t)p & 15);
+        if (c < tot && col * 16 < pre + seg)
+            __builtin_amdgcn_global_load_lds((const glb_void_t*)(p - pre + col * 16), (lds_void_t*)(lds + c0 * 16), 16, 0,
+                                             CPOL);
     }
 }
 

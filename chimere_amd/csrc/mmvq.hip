@@ -55,12 +55,19 @@ constexpr int MMVQ_BLOCKS = 64;
 template <int T>
 constexpr int mmvq_pad() { return T == T_Q4_0 || T == T_Q4_0S || T == T_Q8_0 ? 48 : (T == T_IQ3_S ? 80 : 0); }
 
+// bytes of the GEMV tile: padded rows, or 16-byte spans of unaligned ones
+template <int T>
+constexpr int mmvq_tile() {
+    constexpr int CB = chunk_bytes<T>(MMVQ_BLOCKS), P = mmvq_pad<T>(), S = stage_dw<T>() ? ((CB + 30) & ~15) - CB : 0;
+    return TILE_ROWS * (CB + (P > S ? P : S)) + 16;
+}
+
 // XF32: the f32 entry points' row, quantized by every work-group for itself
 template <int T, int NTOK, bool XF32 = false>
 __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq(MmvqArgs a) {
     constexpr int CBLK = MMVQ_BLOCKS;
-    constexpr int CB = chunk_bytes<T>(CBLK), PAD = mmvq_pad<T>();
-    __shared__ __attribute__((aligned(16))) uint8_t tile[TILE_ROWS * (CB + PAD) + 16];
+    constexpr int PAD = mmvq_pad<T>();
+    __shared__ __attribute__((aligned(16))) uint8_t tile[mmvq_tile<T>()];
     __shared__ XLds xs[NTOK][CBLK];
     __shared__ uint32_t grid[T == T_IQ3_S ? 512 : 1];
 
@@ -121,7 +128,7 @@ __device__ __forceinline__ float quad_of(float v) {
 template <int T, int NG>
 __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_tok(MmvqArgs a) {
     constexpr int CBLK = MMVQ_BLOCKS, CB = chunk_bytes<T>(CBLK), PAD = mmvq_pad<T>();
-    __shared__ __attribute__((aligned(16))) uint8_t tile[TILE_ROWS * (CB + PAD) + 16];
+    __shared__ __attribute__((aligned(16))) uint8_t tile[mmvq_tile<T>()];
     __shared__ __attribute__((aligned(16))) uint8_t xs[4 * NG * XTOK_ROW];
     __shared__ uint32_t grid[T == T_IQ3_S ? 512 : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane >> 2, i = lane & 3;
@@ -141,7 +148,8 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_tok(MmvqArgs a) {
         const int64_t goff = (int64_t)b0 / (QTraits<T>::ELEMS / QK) * QTraits<T>::BYTES;
         const bool al16 = (((uintptr_t)W | (uintptr_t)rb | (uintptr_t)goff | (uintptr_t)seg) & 15) == 0;
         const bool xal = (((uintptr_t)a.x | (uintptr_t)a.x_tok_stride | (uintptr_t)(cb * Q8_1_BYTES)) & 15) == 0;
-        const int lseg = PAD && al16 ? seg + PAD : seg;
+        const bool spans = span_rows<T>(W + goff, rb, nr, seg);
+        const int lseg = spans ? span_stride(seg) : PAD && al16 ? seg + PAD : seg;
         __syncthreads();   // every wave is done with the previous chunk
         bool staged = false;
         if constexpr (CB % 16 == 0)
@@ -150,7 +158,8 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_tok(MmvqArgs a) {
                                                                                              rb, nr, tid);
                 staged = true;
             }
-        if (!staged) stage_rows<stage_dw<T>(), CPOL_STREAM>(tile, W + goff, rb, nr, seg, tid, GEMV_THREADS, lseg);
+        if (spans) stage_row_spans<CPOL_STREAM>(tile, W + goff, rb, nr, seg, tid, GEMV_THREADS);
+        else if (!staged) stage_rows<stage_dw<T>(), CPOL_STREAM>(tile, W + goff, rb, nr, seg, tid, GEMV_THREADS, lseg);
         // tokens past the last repeat it (their sums are not stored); a
         // wave copies whole tokens
 #pragma unroll
@@ -171,13 +180,15 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_mmvq_tok(MmvqArgs a) {
         }
         lds_copy_wait();
         __syncthreads();
-        const uint8_t* row = tile + min(4 * wave + i, nr - 1) * lseg;   // rows past the last repeat it
+        const int ri = min(4 * wave + i, nr - 1);   // rows past the last repeat it
+        const uint8_t* row = tile + ri * lseg;
+        const int pre = spans ? (int)((uintptr_t)(W + goff + ri * rb) & 15) : 0;
 #pragma unroll 1
         for (int bg = 0; bg < cb; bg += SLOTS) {
             const bool in = bg + j < cb;
             const int b = in ? bg + j : cb - 1;
             WBlk w;
-            block_decode<T>(row, b, grid, w);
+            block_decode<T>(row, b, grid, w, pre);
             const float mu = T == T_IQ3_S || T == T_Q4_K || T == T_Q5_K || T == T_Q6_K ? (float)w.mult : 0.0f;
             const float mu2 = T == T_Q6_K ? (float)w.mult2 : 0.0f, mm = (float)w.mmin;
 #pragma unroll

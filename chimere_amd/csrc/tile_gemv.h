@@ -109,11 +109,12 @@ __device__ __forceinline__ void quant_xlds(const float* __restrict__ x, int b0, 
 // lseg) against the chunk's cb decoded activation blocks per token.  KC > 0:
 // a full chunk of a compile-time row stride KC and CBLK blocks (the block loop
 // kept rolled: unrolled it holds more registers and measured slower);
-// CHECK: some of the tile's rows are absent (nr < RG*RPG).
+// CHECK: some of the tile's rows are absent (nr < RG*RPG).  Row r's bytes start
+// (ga + r * gstride) & 15 into its LDS row (0, 0: at its start).
 template <int T, int NT, int RG, int RPG, int CBLK, int KC, bool CHECK>
 __device__ __forceinline__ void tile_compute(const uint8_t* __restrict__ tl, int lseg_rt, int cb_rt,
                                              const XLds* __restrict__ xs, const uint32_t* __restrict__ grid,
-                                             int nr, int ntok, float (&acc)[RPG][NT]) {
+                                             int nr, int ntok, float (&acc)[RPG][NT], uint32_t ga = 0, uint32_t gstride = 0) {
     const int tid = threadIdx.x;
     const int g = tid >> 4, j = tid & 15;
     const int lseg = KC ? KC : lseg_rt, cb = KC ? CBLK : cb_rt;
@@ -128,7 +129,7 @@ __device__ __forceinline__ void tile_compute(const uint8_t* __restrict__ tl, int
                 const int row_i = g + RG * r;
                 if (!CHECK || row_i < nr) {
                     WBlk wb;
-                    block_decode<T>(tl + row_i * lseg, b, grid, wb);
+                    block_decode<T>(tl + row_i * lseg, b, grid, wb, KC ? 0 : (ga + row_i * gstride) & 15);
                     acc[r][0] = wacc<T>(wb, xb, acc[r][0]);
                 }
             }
@@ -142,7 +143,7 @@ __device__ __forceinline__ void tile_compute(const uint8_t* __restrict__ tl, int
 #pragma unroll 1
                 for (int b = j; b < cb; b += SLOTS) {
                     WBlk wb;   // decoded once, used for every token
-                    block_decode<T>(row, b, grid, wb);
+                    block_decode<T>(row, b, grid, wb, KC ? 0 : (ga + row_i * gstride) & 15);
 #pragma unroll
                     for (int t = 0; t < NT; t++) {
                         if (t < ntok) {
@@ -157,12 +158,26 @@ __device__ __forceinline__ void tile_compute(const uint8_t* __restrict__ tl, int
     }
 }
 
+// Whether a tile's row segments go through stage_row_spans: types whose rows may
+// start anywhere (110- and 210-byte superblocks, 17-byte blocks), neither 16-byte
+// aligned nor one aligned run of whole words per row.  By dwords or bytes instead
+// (rows of an odd number of superblocks) Q6_K 4096x4352 took 37.0 us against
+// 10.3, IQ3_S 16384x4352 52.3 against 16.6; as one run, whose LDS rows then are
+// not 4-byte aligned, Q6_K 16384x1280 25.5 us (Q5_K 5.8).
+template <int T>
+__device__ __forceinline__ bool span_rows(const uint8_t* g, int64_t gstride, int nrows, int seg) {
+    return stage_dw<T>() && (((uintptr_t)g | (uintptr_t)gstride | (uintptr_t)seg) & 15) != 0 &&
+           !(gstride == seg && (seg & 3) == 0 && (((uintptr_t)g | (uintptr_t)(seg * nrows)) & 15) == 0);
+}
+
 // One K chunk of tile_gemv (below): blocks [b0, b0 + cb) of the tile's rows.
 // FAST: a full chunk (cb == CBLK) with 16-byte aligned pieces, staged by
 // stage_rows_fixed (the copies issued back to back) and computed with a
 // compile-time row stride and block count; otherwise the general path.
 // XF32: X is the f32 row itself (one token), quantized here (xraw: see quant_xlds).
-template <int T, int NT, int RG, int RPG, int CBLK, int CPOL, int PAD, bool FAST, bool XF32 = false>
+// SPAN: rows that are not 16-byte aligned as spans (span_rows; the tile buffer
+// then needs span_stride bytes per row)
+template <int T, int NT, int RG, int RPG, int CBLK, int CPOL, int PAD, bool FAST, bool XF32 = false, bool SPAN = false>
 __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __restrict__ xs,
                                            const uint32_t* __restrict__ grid, const uint8_t* base1, int n1,
                                            const uint8_t* base2, int n2, int64_t rb, int b0, int cb,
@@ -181,8 +196,11 @@ __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __r
                                       (n2 == 0 || ((uintptr_t)base2 & 15) == 0)))
                          ? seg + PAD
                          : seg;
+    const bool spans = SPAN && n2 == 0 && span_rows<T>(base1 + goff, rb, n1, seg);
     __syncthreads();   // previous users of tile / xs are done
-    if constexpr (FAST) {
+    if (spans) {
+        stage_row_spans<CPOL>(tile, base1 + goff, rb, n1, seg, tid, NTH);
+    } else if constexpr (FAST) {
         static_assert(CB % 16 == 0, "16-byte pieces");
         if (n2 == 0)
             stage_rows_fixed<CB, CB + PAD, 16, RG * RPG, NTH, CPOL, true>(tile, base1 + goff, n1, nullptr, rb, nr, tid);
@@ -212,7 +230,11 @@ __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __r
         else
             tile_compute<T, NT, RG, RPG, CBLK, CB + PAD, true>(tile, 0, 0, xs, grid, nr, ntok, acc);
     } else {
-        tile_compute<T, NT, RG, RPG, CBLK, 0, true>(tile, lseg, cb, xs, grid, nr, ntok, acc);
+        if (spans)
+            tile_compute<T, NT, RG, RPG, CBLK, 0, true>(tile, span_stride(seg), cb, xs, grid, nr, ntok, acc,
+                                                        (uint32_t)(uintptr_t)(base1 + goff), (uint32_t)rb);
+        else
+            tile_compute<T, NT, RG, RPG, CBLK, 0, true>(tile, lseg, cb, xs, grid, nr, ntok, acc);
     }
 }
 
@@ -232,7 +254,8 @@ __device__ __forceinline__ void tile_chunk(uint8_t* __restrict__ tile, XLds* __r
 // FIX: full 16-byte aligned chunks on tile_chunk's FAST path (measured
 // faster for the standalone GEMV, slower -- more registers -- in the MoE
 // kernels' tiles)
-// XF32, xraw: the activation row in f32 (tile_chunk)
+// XF32, xraw: the activation row in f32 (tile_chunk).  With FIX, types of
+// unaligned rows need span_stride bytes per tile row.
 template <int T, int NT, int RG, int RPG, int CBLK = ChunkGeom<T>::BLOCKS, int CPOL = 0, int PAD = 0,
           bool FIX = false, bool XF32 = false>
 __device__ __forceinline__ void tile_gemv(uint8_t* __restrict__ tile, XLds* __restrict__ xs,
@@ -256,7 +279,7 @@ __device__ __forceinline__ void tile_gemv(uint8_t* __restrict__ tile, XLds* __re
             tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, FIXOK, XF32>(tile, xs, grid, base1, n1, base2, n2, rb, b0, CBLK,
                                                                      X, x_tok_stride, toks, ntok, acc, xraw);
         else
-            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, false, XF32>(tile, xs, grid, base1, n1, base2, n2, rb, b0,
+            tile_chunk<T, NT, RG, RPG, CBLK, CPOL, PAD, false, XF32, FIX && stage_dw<T>()>(tile, xs, grid, base1, n1, base2, n2, rb, b0,
                                                                      min(CBLK, nb - b0), X, x_tok_stride, toks, ntok,
                                                                      acc, xraw);
     }

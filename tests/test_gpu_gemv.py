@@ -329,3 +329,25 @@ def test_multi_token_on_matrix_cores(dev, t, nrows, ncols, ntok, off):
     G.gemv_multi(t, dev_t(w, dev), buf[off:], y, nrows, ncols, ntok)
     yo = O.gemv(t, w, xq, ncols, nrows, ntok=ntok, xq_stride=xq.shape[1])
     assert (host(y).view(np.uint32) == np.asarray(yo).reshape(ntok, nrows).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("t", [O.IQ3_S, O.Q6_K, O.MXFP4])
+@pytest.mark.parametrize("nrows,ncols,ntok", [
+    (37, 256, 1), (16, 1280, 1), (50, 4352, 1), (33, 2816, 2), (35, 768, 4), (20, 4352, 8),
+])
+@pytest.mark.parametrize("off", [0, 2, 6])
+def test_gemv_unaligned_rows(dev, t, nrows, ncols, ntok, off):
+    """Rows of an odd number of superblocks (each starts anywhere in a 16-byte
+    granule), whole and ragged chunks, matrices at any even address: bit-exact
+    against the oracle's (L=16, G=1) order."""
+    print(f"unaligned type={t} {nrows}x{ncols} ntok={ntok} off={off}", flush=True)
+    rng = np.random.default_rng(nrows + ncols + ntok + t + off)
+    w = (O.quantize(t, rng.normal(0, 0.02, (nrows, ncols)).astype(np.float32)) if t == O.IQ3_S
+         else npref.rand_kq(t, nrows, ncols, rng))
+    xq = O.quantize_q8_1(rng.standard_normal((ntok, ncols)).astype(np.float32))
+    buf = torch.zeros(w.size + 32, dtype=torch.uint8, device=dev)
+    buf[off:off + w.size] = dev_t(w, dev).reshape(-1)
+    y = torch.zeros(ntok, nrows, dtype=torch.float32, device=dev)
+    G.gemv_multi(t, buf[off:], dev_t(xq, dev), y, nrows, ncols, ntok)
+    yo = O.gemv(t, w, xq, ncols, nrows, ntok=ntok, xq_stride=xq.shape[1])
+    assert (host(y).view(np.uint32) == np.asarray(yo).reshape(ntok, nrows).view(np.uint32)).all()
