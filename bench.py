@@ -14,7 +14,7 @@ of exactly K steps between events, after W warm-up steps.
 Also reported (extra): M=8 IQ3_S layer (config 4, uniform and Zipf routing),
 one token through the IQ3_S layers with a Q8_0 and with a Q5_K shared expert
 (the reference model's types),
-the 512-token Q4_0 prefill chunk (config 5, int8 MFMA), the Q4_0 151936x2048
+the 512-token Q4_0 prefill chunk (config 5, matrix cores), the Q4_0 151936x2048
 head GEMV (config 2), the Q8_0 4096x2048 GEMV (config 1),
 per-kernel times and the roofline of the dominant kernel, and the CPU
 baseline (the C restatement in oracle/, timed on this host).

@@ -240,8 +240,8 @@ void chimere_moe_ffn_decode_stage(const chimere_moe_layer *layer, const float *x
 /* Routed MoE layer for a chunk of ntok >= 1 tokens (prompt prefill).
  * Replaces the reference's per-token loop over the decode MoE during prefill
  * (src/qwen35_model/compute_graph.rs:1787-1800, moe_ffn.rs:1081-1768 per
- * token): tokens are grouped by expert and the expert projections run as int8
- * matrix-core GEMMs.  Same routing and arithmetic per token as
+ * token): tokens are grouped by expert and the expert projections run as
+ * matrix-core GEMMs over exact integer quants.  Same routing and arithmetic per token as
  * chimere_moe_ffn_decode except the fp32 accumulation order of the quantized
  * projections, which is ascending block order (one accumulator per row).
  * Q4_0 / Q8_0 / IQ3_S experts; the shared expert also Q4_K / Q5_K / Q6_K (the
