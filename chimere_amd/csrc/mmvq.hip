@@ -414,9 +414,18 @@ static void gemv_entry(const char* who, int type, const void* W, const void* x, 
 // 4.3; 16384x2048 (1024) Q8_0 10.2 / 9.0, Q4_0 7.9 / 7.1; 65536x2048 (4096)
 // Q4_0 16.1 / 17.7; 8192x4096 (512, two chunks) Q5_K 9.5 / 8.8; 16384x4096
 // (1024, two chunks) Q5_K 12.2 / 13.1.
-static bool f32_one_launch(const float* x, int ncols, int nrows) {
+// Only where the row, the output and the scratch lie apart: the quantizer launch
+// has read all of x before anything is written, so a call may give an output
+// (or, for a short row, a scratch) over its input; in one launch other
+// work-groups still read x when the first ones store.
+static bool f32_one_launch(const float* x, int ncols, int nrows, const float* y, const void* scratch, int ncols_padded) {
     const int64_t wg = (nrows + TILE_ROWS - 1) / TILE_ROWS, chunks = (ncols + MMVQ_BLOCKS * QK - 1) / (MMVQ_BLOCKS * QK);
-    return ((uintptr_t)x & 15) == 0 && wg * chunks <= 1024;   // 16-byte loads of x
+    if (((uintptr_t)x & 15) != 0 || wg * chunks > 1024) return false;   // 16-byte loads of x
+    auto apart = [](const void* p, int64_t np, const void* q, int64_t nq) {
+        return (uintptr_t)p + (uintptr_t)np <= (uintptr_t)q || (uintptr_t)q + (uintptr_t)nq <= (uintptr_t)p;
+    };
+    const int64_t xb = (int64_t)ncols * 4, yb = (int64_t)nrows * 4, sb = (int64_t)(ncols_padded / QK) * Q8_1_BYTES;
+    return apart(x, xb, y, yb) && apart(x, xb, scratch, sb) && apart(y, yb, scratch, sb);
 }
 
 static void gemv_f32_entry(const char* who, int type, const void* W, const float* x, float* y,
@@ -427,7 +436,7 @@ static void gemv_f32_entry(const char* who, int type, const void* W, const float
         return;
     }
     if (!check_gemv(who, type, W, scratch, y, ncols, nrows, ncols_padded / 32, 1)) return;
-    if (f32_one_launch(x, ncols, nrows)) {
+    if (f32_one_launch(x, ncols, nrows, y, scratch, ncols_padded)) {
         MmvqArgs a{(const uint8_t*)W, (const uint8_t*)x, y, ncols, nrows, 1, 0, nrows, nullptr, 0, 0, 0,
                    (uint8_t*)scratch, ncols_padded / 32};
         launch_mmvq_f32(type, a, s);

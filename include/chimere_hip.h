@@ -79,8 +79,9 @@ void chimere_mmvq_q4_0(const void *weights, const void *input_q8, float *output,
 void chimere_mmvq_q4_0_sform(const void *weights, const void *input_q8, float *output,
                              int ncols, int nrows, int nrows_y_padded, hipStream_t stream);
 
-/* Fused F32 -> Q8_1 -> GEMV (ggml_cuda_gemv.cu:302-387): quantizes input_f32
- * into q8_scratch (pad(ncols,512)/32*36 bytes) then runs the GEMV. */
+/* Fused F32 -> Q8_1 -> GEMV (ggml_cuda_gemv.cu:302-387): the GEMV of
+ * input_f32's Q8_1 blocks, which q8_scratch (pad(ncols,512)/32*36 bytes) holds
+ * afterwards.  output may overlap input_f32 (the input is read first). */
 void chimere_mmvq_iq3s_f32(const void *weights, const float *input_f32, float *output,
                            int ncols, int nrows, int ncols_padded, void *q8_scratch,
                            hipStream_t stream);

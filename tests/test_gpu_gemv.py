@@ -351,3 +351,55 @@ def test_gemv_unaligned_rows(dev, t, nrows, ncols, ntok, off):
     G.gemv_multi(t, buf[off:], dev_t(xq, dev), y, nrows, ncols, ntok)
     yo = O.gemv(t, w, xq, ncols, nrows, ntok=ntok, xq_stride=xq.shape[1])
     assert (host(y).view(np.uint32) == np.asarray(yo).reshape(ntok, nrows).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("t", [O.Q8_0, O.Q4_0, O.Q5_K])
+@pytest.mark.parametrize("n,shift", [(2048, 0), (2048, 1024), (2048, -1024), (2304, 0), (4096, 0), (8192, 0)])
+def test_f32_gemv_output_over_input(dev, t, n, shift):
+    """A square projection whose output is its input's buffer (shift 0) or a
+    view that overlaps half of it: the bits of the call with its own output.
+    Disjoint buffers of all sizes but the last take a single launch, in which
+    later work-groups would read outputs that earlier ones stored."""
+    print(f"f32 output over input type={t} n={n} shift={shift}", flush=True)
+    rng = np.random.default_rng(n + t)
+    # random blocks, f16 scales below 1
+    w = torch.randint(0, 60, (n * O.row_bytes(t, n),), dtype=torch.uint8, device=dev,
+                      generator=torch.Generator(device=dev).manual_seed(t))
+    x = dev_t(rng.standard_normal(n).astype(np.float32), dev)
+    fn = {O.Q8_0: G.ggml_gpu_gemv_q8_0_f32, O.Q4_0: G.ggml_gpu_gemv_q4_0_f32, O.Q5_K: G.ggml_gpu_gemv_q5k_f32}[t]
+    scratch = torch.empty(G.q8_1_row_bytes(n), dtype=torch.uint8, device=dev)
+    want = torch.zeros(n, device=dev)
+    fn(w, x, want, scratch, n, n)
+    want = host(want).view(np.uint32)
+    buf = torch.zeros(n + 2 * abs(shift), device=dev)
+    xv = buf[abs(shift):abs(shift) + n]
+    yv = buf[abs(shift) + shift:abs(shift) + shift + n]
+    for _ in range(3):
+        xv.copy_(x)
+        fn(w, xv, yv, scratch, n, n)
+        assert (host(yv).view(np.uint32) == want).all()
+
+
+@pytest.mark.parametrize("where", ["row", "output"])
+def test_f32_gemv_scratch_over_row_or_output(dev, where):
+    """One 32-element block: a scratch that starts where the row does (the
+    quantizer's wave reads the block before it writes), and an output over the
+    scratch's zero blocks past the row's own (which no GEMV reads): the bits of
+    the call with buffers of its own."""
+    import ctypes as C
+    from chimere_amd._lib import check, lib
+    n, nrows, pad = 32, 2048, 32 if where == "row" else 512
+    rng = np.random.default_rng(7)
+    w = dev_t(O.quantize(O.Q8_0, rng.normal(0, 0.02, (nrows, n)).astype(np.float32)), dev)
+    x = rng.standard_normal(n).astype(np.float32)
+    want = np.asarray(O.gemv(O.Q8_0, host(w), O.quantize_q8_1(x), n, nrows)).reshape(-1)
+    buf = torch.zeros(nrows + 1024, device=dev)
+    # floats: row, scratch, output
+    xo, so, yo = (0, 0, 256) if where == "row" else (nrows + 512, 0, 9)
+    for _ in range(3):
+        buf.zero_()
+        buf[xo:xo + n] = dev_t(x, dev)
+        p = [C.c_void_p(buf.data_ptr() + 4 * o) for o in (xo, yo, so)]
+        lib().chimere_mmvq_q8_0_f32(C.c_void_p(w.data_ptr()), p[0], p[1], n, nrows, pad, p[2], G._stream())
+        check()
+        assert (host(buf[yo:yo + nrows]).view(np.uint32) == want.view(np.uint32)).all()
