@@ -73,7 +73,6 @@ struct PfArgs {
 // (its 34-byte blocks)
 template <int T>
 constexpr int pf_ch() { return T == T_Q8_0 ? 4 : 8; }
-constexpr int PF_XB = 4;         // blocks of the activation rows per LDS stage
 // bytes of a chunk
 template <int T>
 constexpr int pf_cb() { return QTraits<T>::ELEMS == 256 ? QTraits<T>::BYTES : pf_ch<T>() * QTraits<T>::BYTES; }
@@ -315,12 +314,12 @@ struct PfLds {
 // (vmcnt counts in order) with the weight chunk still in flight: its HBM round
 // trip has a whole chunk of work to hide behind.  WDB false: one weight stage
 // over the memory of both (shared-expert rows wider than a stage).
-template <int T, int MT, bool WDB, class Done>
+template <int T, int MT, int XB, bool WDB, class Done>
 __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const uint8_t* w1, int64_t rb, int ns,
                                         int64_t sstride, int nbk,
                                         const _Float16* xh, const uint32_t* xd, const float* xs, const int* list,
                                         int first, int np, const uint32_t* grid, Done done) {
-    constexpr int NTN = 2, CH = pf_ch<T>(), CB = pf_cb<T>(), SL = pf_sl<T>(), XB = PF_XB, SPC = CH / XB;
+    constexpr int NTN = 2, CH = pf_ch<T>(), CB = pf_cb<T>(), SL = pf_sl<T>(), SPC = CH / XB;
     constexpr int NSLOT = pf_row<T>(PF_ROWS) / 16, NWG = (NSLOT + 63) / 64, NIT = (NWG + 3) / 4;
     constexpr int KT = 4 / MT;   // blocks whose scale products one 4-block instruction makes
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c = lane & 15;
@@ -558,17 +557,22 @@ constexpr bool pf_single() { return MT == 2; }
 // bytes of a weight stage next to experts of type TE: a shared type of at most
 // 10 slots per row has two stages too, a wider one (and the K-quants) a single
 // stage over both; with one weight stage it holds either
-template <int TE, int TS, int MT>
+template <int TE, int TS, bool ONE>
 constexpr int pf_wst2() {
-    return pf_wst<TS>() > pf_wst<TE>() && (pf_single<MT>() || (pf_sl<TS>() <= 10 && !pf_kq<TS>())) ? pf_wst<TS>()
-                                                                                                   : pf_wst<TE>();
+    return pf_wst<TS>() > pf_wst<TE>() && (ONE || (pf_sl<TS>() <= 10 && !pf_kq<TS>())) ? pf_wst<TS>() : pf_wst<TE>();
 }
-template <int T, int TE, int TS, int MT>
-constexpr bool pf_wdb() { return !pf_single<MT>() && pf_wst<T>() <= pf_wst2<TE, TS, MT>(); }
-template <int MT>
-constexpr int pf_xst() { return MT * PF_XB * 1024; }
-template <int MT>
-constexpr int pf_dst() { return 16 * MT * PF_XB; }   // words of a scale stage
+template <int T, int TE, int TS, bool ONE>
+constexpr bool pf_wdb() { return !ONE && pf_wst<T>() <= pf_wst2<TE, TS, ONE>(); }
+// Blocks of the activation rows per LDS stage, M tiles of 16 pairs at a time:
+// a whole chunk (one barrier less) where two weight stages leave two
+// work-groups per CU either way, that is, for the tiles of up to 32 pairs of the
+// 64-pair kernels (with four blocks, 800 tokens: IQ3_S + Q6_K 268 -> 274 us,
+// IQ3_S + Q8_0 254 -> 258, Q4_0 235 -> 238)
+template <int T, int M, bool ONE>
+constexpr int pf_xb() { return pf_ch<T>() == 8 && M == 2 && !ONE ? 8 : 4; }
+// blocks x 16-pair tiles of an activation stage
+template <int MT, bool ONE>
+constexpr int pf_xu() { return MT == 2 && !ONE ? 16 : 4 * MT; }
 
 // Work-group -> (slot of the tile list, slice of rows).  The hardware deals
 // work-groups to the 8 XCDs round-robin; slots 8 g + x are XCD x's, and the
@@ -583,10 +587,11 @@ __device__ __forceinline__ int4 pf_place(const PfArgs& a, int nslice, int& sl) {
 // LDS arrays of a work-group
 #define PF_LDS_ARRAYS                                                                                       \
     constexpr bool IQ = TE == T_IQ3_S || TS == T_IQ3_S, KQ = pf_kq<TS>();                                   \
-    __shared__ __attribute__((aligned(16))) uint8_t smem[(pf_single<MT>() ? 1 : 2) * pf_wst2<TE, TS, MT>() + 2 * pf_xst<MT>()];         \
-    __shared__ __attribute__((aligned(16))) uint32_t sd[(KQ ? 4 : 2) * pf_dst<MT>()];                           \
+    constexpr int NW = ONE ? 1 : 2, XU = pf_xu<MT, ONE>(), WST = pf_wst2<TE, TS, ONE>();                     \
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NW * WST + 2 * XU * 1024];                         \
+    __shared__ __attribute__((aligned(16))) uint32_t sd[(KQ ? 4 : 2) * XU * 16];                            \
     __shared__ __attribute__((aligned(16))) uint32_t grid[IQ ? 1024 : 1];                                   \
-    const PfLds L{smem, sd, pf_wst2<TE, TS, MT>(), pf_xst<MT>(), pf_dst<MT>(), pf_single<MT>() ? 1 : 2};                                      \
+    const PfLds L{smem, sd, WST, XU * 1024, XU * 16, NW};                                                   \
     /* the codebook, one kilobyte per wave; landed with the first weight chunk */                           \
     if constexpr (IQ)                                                                                       \
         copy16_lds_untracked((const uint4*)c_iq3s_hgrid.w + threadIdx.x, (uint4*)grid + (threadIdx.x & ~63u))
@@ -620,7 +625,8 @@ __device__ __forceinline__ void pf_dispatch(const int4& ti, bool sh, Run run) {
 // epilogue, measured slower: 512 tokens Q4_0 108 -> 118 and 144 us -- fewer
 // work-groups, and the loop's state held across the epilogue.)
 template <int TE, int TS, int MT>
-__global__ __launch_bounds__(PF_THREADS, MT == 2 ? 3 : 2) void k_pf_gate_up(PfArgs a) {
+__global__ __launch_bounds__(PF_THREADS, pf_single<MT>() ? 3 : 2) void k_pf_gate_up(PfArgs a) {
+    constexpr bool ONE = pf_single<MT>();
     int sl;
     const int4 ti = pf_place(a, a.F / 64, sl);
     if (ti.z == 0) return;
@@ -634,7 +640,7 @@ __global__ __launch_bounds__(PF_THREADS, MT == 2 ? 3 : 2) void k_pf_gate_up(PfAr
     pf_dispatch<TE, TS, MT, 4>(ti, sh, [&](auto ttag, auto mtag, int start, int np) {
         constexpr int T = decltype(ttag)::value, M = decltype(mtag)::value;
         const int64_t rb = row_bytes(T, a.H);
-        pf_gemm<T, M, pf_wdb<T, TE, TS, MT>()>(L, g + f0 * rb, u + f0 * rb, rb, 1, 64 * rb, a.H / QK, a.xh, a.xd,
+        pf_gemm<T, M, pf_xb<T, M, ONE>(), pf_wdb<T, TE, TS, ONE>()>(L, g + f0 * rb, u + f0 * rb, rb, 1, 64 * rb, a.H / QK, a.xh, a.xd,
                                            a.xs, a.stok, start, np, grid, [&](int, float (&acc)[2][M][4]) {
             // wave w has gate and up of rows f0 + 16 w + c: half a block of h.
             // Q8_1 as k_quantize_q8_1: the halves' maxima (K-quants: quant
@@ -707,7 +713,8 @@ __global__ __launch_bounds__(PF_THREADS, MT == 2 ? 3 : 2) void k_pf_gate_up(PfAr
 // Q8_0 130 -> 121 us.
 constexpr int PF_DN_NS = 2;
 template <int TE, int TS, int MT>
-__global__ __launch_bounds__(PF_THREADS, MT == 2 ? 3 : 2) void k_pf_down(PfArgs a) {
+__global__ __launch_bounds__(PF_THREADS, pf_single<MT>() ? 3 : 2) void k_pf_down(PfArgs a) {
+    constexpr bool ONE = pf_single<MT>();
     int sl;
     const int4 ti = pf_place(a, a.H / (PF_ROWS * PF_DN_NS), sl);
     if (ti.z == 0) return;
@@ -724,7 +731,7 @@ __global__ __launch_bounds__(PF_THREADS, MT == 2 ? 3 : 2) void k_pf_down(PfArgs 
         for (int m = 0; m < M; m++)
 #pragma unroll
             for (int i = 0; i < 4; i++) prs[m][i] = a.spairs[start + min(16 * m + 4 * q + i, np - 1)];
-        pf_gemm<T, M, pf_wdb<T, TE, TS, MT>()>(L, d + r0 * rb, d + (r0 + 64) * rb, rb, PF_DN_NS, PF_ROWS * rb, a.F / QK,
+        pf_gemm<T, M, pf_xb<T, M, ONE>(), pf_wdb<T, TE, TS, ONE>()>(L, d + r0 * rb, d + (r0 + 64) * rb, rb, PF_DN_NS, PF_ROWS * rb, a.F / QK,
                                            a.hh, a.hd, a.hs, nullptr, start, np, grid, [&](int s, float (&acc)[2][M][4]) {
             const int r = r0 + s * PF_ROWS + 16 * wave + c;
 #pragma unroll
