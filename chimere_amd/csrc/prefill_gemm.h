@@ -551,9 +551,16 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
 // which hides a chunk's copies better than a second stage (512 tokens Q4_0
 // gate/up 110 -> 104 us, down 61 -> 55; IQ3_S + Q5_K gate/up 128 -> 117).  16
 // pairs have three work-groups with two stages (one: 45 tokens IQ3_S + Q5_K
-// 76 -> 82 us), 64 pairs two either way, by their registers.
-template <int MT>
-constexpr bool pf_single() { return MT == 2; }
+// 76 -> 82 us), 64 pairs two either way, by their registers.  Not for the down
+// launch next to a shared type of two-part blocks: its loop holds up to 199
+// registers, and in a third of the register file Q4_K / Q5_K / Q6_K spilled 25 /
+// 34 / 36 of them (512 tokens, one stage / two: Q4_0 + Q6_K 219 / 203 us, Q4_0 +
+// Q5_K 213 / 201, IQ3_S + Q6_K 227 / 218, IQ3_S + Q5_K 224 / 216, IQ3_S + Q4_K
+// 220 / 216; 16 pairs at a time in one stage are 1-2 % faster still with IQ3_S
+// experts but 17 % slower for 256 tokens at H = F = 1024).  The gate/up launch
+// (at most 7 spilled) keeps one: with two, IQ3_S + Q6_K 220 us, + Q5_K 221, + Q4_K 221.
+template <int TS, int MT, bool DOWN>
+constexpr bool pf_single() { return MT == 2 && !(DOWN && (pf_kq<TS>() || TS == T_Q6_K)); }
 // bytes of a weight stage next to experts of type TE: a shared type of at most
 // 10 slots per row has two stages too, a wider one (and the K-quants) a single
 // stage over both; with one weight stage it holds either
@@ -565,8 +572,8 @@ template <int T, int TE, int TS, bool ONE>
 constexpr bool pf_wdb() { return !ONE && pf_wst<T>() <= pf_wst2<TE, TS, ONE>(); }
 // Blocks of the activation rows per LDS stage, M tiles of 16 pairs at a time:
 // a whole chunk (one barrier less) where two weight stages leave two
-// work-groups per CU either way, that is, for the tiles of up to 32 pairs of the
-// 64-pair kernels (with four blocks, 800 tokens: IQ3_S + Q6_K 268 -> 274 us,
+// work-groups per CU either way: in the tiles of up to 32 pairs of the 64-pair
+// kernels, and in the 32-pair kernels of two weight stages (with four blocks, 800 tokens: IQ3_S + Q6_K 268 -> 274 us,
 // IQ3_S + Q8_0 254 -> 258, Q4_0 235 -> 238)
 template <int T, int M, bool ONE>
 constexpr int pf_xb() { return pf_ch<T>() == 8 && M == 2 && !ONE ? 8 : 4; }
@@ -625,8 +632,8 @@ __device__ __forceinline__ void pf_dispatch(const int4& ti, bool sh, Run run) {
 // epilogue, measured slower: 512 tokens Q4_0 108 -> 118 and 144 us -- fewer
 // work-groups, and the loop's state held across the epilogue.)
 template <int TE, int TS, int MT>
-__global__ __launch_bounds__(PF_THREADS, pf_single<MT>() ? 3 : 2) void k_pf_gate_up(PfArgs a) {
-    constexpr bool ONE = pf_single<MT>();
+__global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, false>() ? 3 : 2)) void k_pf_gate_up(PfArgs a) {
+    constexpr bool ONE = pf_single<TS, MT, false>();
     int sl;
     const int4 ti = pf_place(a, a.F / 64, sl);
     if (ti.z == 0) return;
@@ -713,8 +720,8 @@ __global__ __launch_bounds__(PF_THREADS, pf_single<MT>() ? 3 : 2) void k_pf_gate
 // Q8_0 130 -> 121 us.
 constexpr int PF_DN_NS = 2;
 template <int TE, int TS, int MT>
-__global__ __launch_bounds__(PF_THREADS, pf_single<MT>() ? 3 : 2) void k_pf_down(PfArgs a) {
-    constexpr bool ONE = pf_single<MT>();
+__global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, true>() ? 3 : 2)) void k_pf_down(PfArgs a) {
+    constexpr bool ONE = pf_single<TS, MT, true>();
     int sl;
     const int4 ti = pf_place(a, a.H / (PF_ROWS * PF_DN_NS), sl);
     if (ti.z == 0) return;
