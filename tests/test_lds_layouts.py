@@ -3,9 +3,9 @@
 * stage_rows with an LDS row stride above the row bytes (chimere_amd/csrc/
   common.h), as the GEMV tile uses it (chimere_amd/csrc/tile_gemv.h,
   mmvq.hip: Q4_0 / Q8_0 / IQ3_S chunks, row padding 48 / 48 / 80 bytes);
-* the two-stage prefill copy loop (chimere_amd/csrc/prefill.hip, pf_gemm_k):
-  weight rows in slots of pf_lds_row_al bytes (IQ3_S 128 -> 144) and the
-  tile's activation rows in slots of 304 bytes (8 Q8_1 blocks + 16).
+* stage_row_spans with the tile's row stride for unaligned rows;
+* the prefill GEMMs' stages (chimere_amd/csrc/prefill_gemm.h) and the slots of
+  the plan's tile list (prefill.hip).
 
 The slot -> (row, column) arithmetic is transcribed from the kernels.  Every
 16-byte piece of every row must be written exactly once, no write may leave
@@ -15,8 +15,8 @@ read may touch) must stay inside the buffer."""
 import pytest
 
 QK = 32
-BYTES = {"q4_0": 18, "q8_0": 34, "iq3s": 110, "q6k": 210}
-ELEMS = {"q4_0": 32, "q8_0": 32, "iq3s": 256, "q6k": 256}
+BYTES = {"q4_0": 18, "q8_0": 34, "iq3s": 110, "q6k": 210, "mxfp4": 17}
+ELEMS = {"q4_0": 32, "q8_0": 32, "iq3s": 256, "q6k": 256, "mxfp4": 32}
 
 
 def chunk_bytes(t, blocks):
@@ -68,60 +68,218 @@ def test_gemv_tile_padded_rows(t, pad, ncols):
             assert (nr - 1) * lseg + seg + 4 <= buf
 
 
-PF_CHUNK, PF_TILE, PF_THREADS = 8, 16, 256
-PF_XROW, PF_XROW_AL = PF_CHUNK * 36, PF_CHUNK * 36 + 16
+# ---- prefill_gemm.h: the work-group's LDS and the copies into it
+
+# blocks and bytes of a chunk
+PF = {"q4_0": (8, 144), "q8_0": (4, 136), "iq3s": (8, 110), "q4k": (8, 144), "q5k": (8, 176), "q6k": (8, 210)}
+EXPERT, SHARED, KQ = ("q4_0", "q8_0", "iq3s"), tuple(PF), ("q4k", "q5k")
+PF_ROWS = 128
 
 
-def pf_lds_row(t):
-    return {"iq3s": 128, "q6k": 224}.get(t, chunk_bytes(t, PF_CHUNK))
+def pf_sl(t):
+    return (PF[t][1] + 14 + 15) // 16 + (t in ("iq3s", "q6k", "q5k"))
 
 
-def pf_lds_row_al(t):
-    r = pf_lds_row(t)
-    return r + 16 if r % 128 == 0 else r
+def pf_skew(t):
+    return pf_sl(t) % 2 == 0
 
 
-@pytest.mark.parametrize("t,NR,n0", [("q4_0", 128, 64), ("q8_0", 128, 64), ("iq3s", 128, 64), ("iq3s", 128, 128),
-                                     ("q4_0", 128, 128), ("q6k", 128, 64), ("q6k", 128, 128)])
-def test_prefill_two_stage_padded_slots(t, NR, n0):
-    CBL, CBLP = pf_lds_row(t), pf_lds_row_al(t)
-    PCB, PCBP, PER, PERP = CBL // 16, CBLP // 16, PF_XROW // 16, PF_XROW_AL // 16
-    TW = NR * PCBP
-    TWP = (TW + 63) & ~63
-    TOT = TWP + PF_TILE * PERP
-    wbuf = NR * CBLP + 16          # pf_wst
-    xbuf = PF_TILE * PF_XROW_AL    # PF_XST
-    NIT = (TOT + PF_THREADS - 1) // PF_THREADS
-    wseen, xseen = set(), set()
-    for tid in range(PF_THREADS):
-        lane, wave = tid & 63, tid >> 6
-        for k in range(NIT):
-            c0 = wave * 64 + k * PF_THREADS
-            cc = c0 + lane
-            if c0 < TWP:
-                if cc < TW:
-                    row, col = divmod(cc, PCBP)
-                    if col < PCB:
-                        dst = c0 * 16 + lane * 16
-                        assert dst == row * CBLP + col * 16 and dst + 16 <= wbuf
-                        assert (row, col) not in wseen
-                        wseen.add((row, col))
-            elif c0 < TOT:
-                xc = cc - TWP
-                if xc < PF_TILE * PERP:
-                    r, col = divmod(xc, PERP)
-                    if col < PER:
-                        dst = (c0 - TWP) * 16 + lane * 16
-                        assert dst == r * PF_XROW_AL + col * 16 and dst + 16 <= xbuf
-                        assert (r, col) not in xseen
-                        xseen.add((r, col))
-    assert len(wseen) == NR * PCB and len(xseen) == PF_TILE * PER
-    # readers: the last row's chunk (at most 14 bytes into its span for IQ3_S
-    # and Q6_K) plus a 4-byte unaligned read; the activation metadata / fragments
-    span_off = max(c * chunk_bytes(t, PF_CHUNK) % 16 for c in range(16))   # 110- / 210-byte chunks: 14
-    assert span_off + chunk_bytes(t, PF_CHUNK) <= CBL   # the chunk fits its span
-    assert (NR - 1) * CBLP + span_off + chunk_bytes(t, PF_CHUNK) + 4 <= wbuf
-    assert (PF_TILE - 1) * PF_XROW_AL + (PF_CHUNK - 1) * 36 + 36 <= xbuf
+def pf_row(t, r):
+    return (r * pf_sl(t) + (r >> 2 if pf_skew(t) else 0)) * 16
+
+
+def pf_wst(t):
+    return pf_row(t, PF_ROWS) + 16
+
+
+def pf_furthest(t, s):
+    """End of the furthest LDS read of a row whose chunk starts at s (three whole
+    words from the word that holds a field's first byte, two for a 32-bit one)."""
+    w3, w2 = (lambda a: (a & ~3) + 12), (lambda a: (a & ~3) + 8)
+    return max({"q4_0": lambda: [w3(s + 2 + 8 + 18 * 7), w3(s + 2 + 8 + 18 * 6)],
+                "q8_0": lambda: [w3(s + 2 + 24 + 34 * 3), w3(s + 2 + 24 + 34 * 2)],
+                "iq3s": lambda: [w2(s + 106), w2(s + 70), s + 74 + 4 * 7 + 4],
+                "q4k": lambda: [w3(s + 16 + 24) + 96, w2(s + 12)],
+                "q5k": lambda: [w3(s + 48 + 24) + 96, w2(s + 20 + 24)],
+                "q6k": lambda: [w2(s + 128 + 32 + 24 + 4), s + 210]}[t]())
+
+
+def pf_weight_pieces(t):
+    """(instruction, lane) -> (row, column) of one chunk's copies, and each wave's
+    number of instructions."""
+    sl = pf_sl(t)
+    nwg = (pf_row(t, PF_ROWS) // 16 + 63) // 64
+    out = {}
+    for g in range(nwg):
+        for lane in range(64):
+            cc = g * 64 + lane
+            if pf_skew(t):
+                g4, rem = divmod(cc, 4 * sl + 1)
+                r, col = 4 * g4 + rem // sl, (rem % sl if rem < 4 * sl else sl)
+            else:
+                r, col = divmod(cc, sl)
+            out[g, lane] = (r, col) if r < PF_ROWS and col < sl else None
+    nwi = [(nwg - wave + 3) // 4 for wave in range(4)]
+    assert nwi == [len([g for g in range(nwg) if g % 4 == w]) for w in range(4)]
+    return nwg, out
+
+
+@pytest.mark.parametrize("t", SHARED)
+def test_prefill_weight_stage(t):
+    """Rows whose chunks start at any even place of a 16-byte granule: every piece
+    of every row's span is copied once to its row's slots, inside the stage; every
+    copy instruction of a wave has an active lane (the waits count them); no read
+    of a row leaves the stage or the bytes copied for it, but for the words'
+    padding, which is inside the stage."""
+    cb = PF[t][1]
+    nwg, pieces = pf_weight_pieces(t)
+    for phase, stride in [(p, s) for p in range(0, 16, 2) for s in (0, 2, 14)]:
+        seen, active = set(), {g: 0 for g in range(nwg)}
+        for (g, lane), rc in pieces.items():
+            if rc is None:
+                continue
+            r, col = rc
+            pre = (phase + r * stride) % 16
+            if col * 16 < pre + cb:
+                active[g] += 1
+                dst = g * 1024 + lane * 16
+                assert dst == pf_row(t, r) + 16 * col and dst + 16 <= pf_wst(t) - 16
+                assert (r, col) not in seen
+                seen.add((r, col))
+        assert all(active.values())
+        assert seen == {(r, c) for r in range(PF_ROWS) for c in range(((phase + r * stride) % 16 + cb + 15) // 16)}
+        for r in range(PF_ROWS):
+            s = pf_row(t, r) + (phase + r * stride) % 16
+            assert s + cb <= pf_row(t, r) + 16 * pf_sl(t)
+            assert pf_furthest(t, s) <= pf_wst(t)
+
+
+def pf_work_group(launch, te, ts, mt):
+    """(stages, bytes of a weight stage, 16-pair x block units of an activation
+    stage) of a kernel's LDS, and its runs: (type, pair tiles, activation blocks
+    per stage, two weight stages)."""
+    one = mt == 2 and not (launch == "down" and ts in KQ + ("q6k",))
+    wide = pf_wst(ts) > pf_wst(te) and (one or (pf_sl(ts) <= 10 and ts not in KQ))
+    wst2 = pf_wst(ts if wide else te)
+    xu = 16 if mt == 2 and not one else 4 * mt
+    runs = []
+    for t in {te, ts}:
+        most = 2 if t == "q6k" else (4 if launch == "gate_up" else 2) if t in KQ else 4
+        m = min(mt, most)
+        for k in {m} if m < mt else {mt, max(1, mt // 2)}:
+            runs.append((t, k, 8 if PF[t][0] == 8 and k == 2 and not one else 4, not one and pf_wst(t) <= wst2))
+    return 1 if one else 2, wst2, xu, runs
+
+
+@pytest.mark.parametrize("launch", ["gate_up", "down"])
+@pytest.mark.parametrize("mt", [1, 2, 4])
+def test_prefill_work_group_lds(launch, mt):
+    """Every type x tile size run by a kernel fits its LDS: the weight stages, the
+    activation and scale stages, the wave's copies of the row list (in the second
+    activation stage) and the epilogue's exchange (in the scale stages)."""
+    for te, ts in [(te, ts) for te in EXPERT for ts in SHARED]:
+        nw, wst2, xu, runs = pf_work_group(launch, te, ts, mt)
+        sd = (4 if ts in KQ else 2) * xu * 16                      # words
+        total = nw * wst2 + 2 * xu * 1024 + 4 * sd + (4096 if "iq3s" in (te, ts) else 16)
+        assert total <= 160 * 1024 // (3 if mt == 2 and nw == 1 else 2)
+        for t, m, xb, wdb in runs:
+            assert 2 * pf_wst(t) <= nw * wst2 if wdb else pf_wst(t) <= nw * wst2
+            assert PF[t][0] % xb == 0 and m * xb <= xu
+            assert 16 * m * xb <= xu * 16
+            assert 4 * 64 * 4 <= xu * 1024 and 16 * m <= 64        # the list holds 64 rows
+            assert 4 * 16 * m <= sd
+
+
+@pytest.mark.parametrize("mt,xb", [(1, 4), (2, 4), (2, 8), (4, 4)])
+def test_prefill_activation_stage(mt, xb):
+    """The pieces that the copies leave in an activation stage, and the words in a
+    scale stage, are those the lanes read: each piece copied once."""
+    nxp, nxb = (mt // 2, xb // 2) if mt > 1 else (1, xb // 4)
+    lds, sc = {}, {}
+    for wave in range(4):
+        for lane in range(64):
+            for j in range(nxp):
+                grp, r = (wave + 4 * j if mt > 1 else wave & 1), lane >> 3
+                for k in range(nxb):
+                    unit = xb // 2 * (wave + 4 * j) + k if mt > 1 else xb // 2 * (wave & 1) + nxb * (wave >> 1) + k
+                    off = (0 if mt > 1 else 128 * nxb * (wave >> 1)) + 16 * ((lane & 7) ^ r) + 128 * k
+                    at = unit * 1024 + lane * 16
+                    assert at not in lds and at + 16 <= mt * xb * 1024
+                    lds[at] = (8 * grp + r, off)              # pair, byte of its row's stage
+    assert sorted(lds.values()) == [(p, o) for p in range(16 * mt) for o in range(0, 64 * xb, 16)]
+    for lane in range(16 * mt):
+        for k in range(xb // 4):
+            for i in range(4):
+                sc[64 * mt * k + 4 * lane + i] = (lane, 4 * k + i)
+    assert sorted(sc) == list(range(16 * mt * xb))
+    kt = 4 // mt
+    for q in range(4):
+        for c in range(16):
+            xo = (c >> 3) * (512 * xb) + (c & 7) * 128 + (q ^ (c & 7)) * 16
+            for b in range(xb):
+                for m in range(mt):
+                    at = m * (1024 * xb) + (b >> 1) * 1024 + (xo ^ 64 if b & 1 else xo)
+                    assert lds[at] == (16 * m + c, 64 * b + 16 * q)
+                    for i in range(4):
+                        assert sc[(16 * m + 4 * q + i) * 4 + 64 * mt * (b >> 2) + (b & 3)] == (16 * m + 4 * q + i, b)
+                if b % kt == 0:
+                    assert sc[64 * mt * (b >> 2) + (b & 3) + (16 * (q % mt) + c) * 4 + q // mt] == \
+                        (16 * (q % mt) + c, b + q // mt)
+
+
+@pytest.mark.parametrize("tp", [16, 32, 64])
+@pytest.mark.parametrize("E,K,T", [(1, 1, 1), (4, 2, 33), (8, 8, 130), (256, 8, 45), (256, 8, 512), (300, 12, 70),
+                                   (1024, 16, 65)])
+def test_prefill_tile_slots(tp, E, K, T):
+    """The plan's tiles (experts' in contiguous eighths, one per XCD, after the
+    shared expert's) have a slot each inside the list, however the router deals
+    the pairs."""
+    import random
+    rng = random.Random(E * K + T)
+    slots = lambda n: ((T * K + T) // n + E + 1 + 14 + 7) // 8 * 8  # noqa: E731
+    assert slots(tp) <= slots(16)                               # the workspace's size
+    for shared in (False, True):
+        for case in range(8):
+            counts = [0] * E
+            for _ in range(T):
+                hot = range(K) if case == 0 else sorted(rng.sample(range(E), K))
+                for e in hot:
+                    counts[e] += 1
+            if case == 1:                                       # one pair left over everywhere it can be
+                counts = [tp + 1 if i < T * K // (tp + 1) else 0 for i in range(E)]
+            ne = sum((c + tp - 1) // tp for c in counts)
+            nsh = (T + tp - 1) // tp if shared else 0
+            per, persh = max((ne + 7) >> 3, 1), (nsh + 7) >> 3
+            used = list(range(nsh)) + [8 * (persh + t - t // per * per) + t // per for t in range(ne)]
+            assert len(set(used)) == ne + nsh and max(used, default=0) < slots(tp)
+
+
+@pytest.mark.parametrize("t", ["iq3s", "q6k", "mxfp4"])
+def test_gemv_row_spans(t):
+    """stage_row_spans (common.h) into the GEMV tile (mmvq_tile, mmvq.hip): whole
+    and ragged chunks, rows at any place of a granule (MXFP4: odd ones too)."""
+    pad = {"iq3s": 80}.get(t, 0)
+    cb = chunk_bytes(t, 64)
+    tile = 16 * (cb + max(pad, ((cb + 30) & ~15) - cb)) + 16
+    for blocks in {"mxfp4": range(1, 65, 7)}.get(t, range(8, 65, 8)):
+        seg = chunk_bytes(t, blocks)
+        ss = (seg + 30) & ~15
+        per = ss >> 4
+        for rb in {seg, 3 * seg, seg + 7 * BYTES[t]}:
+            for phase in range(0, 16, 1 if t == "mxfp4" else 2):
+                for nr in (16, 5, 1):
+                    seen = {}
+                    for c in range(per * nr):
+                        r, col = divmod(c, per)
+                        pre = (phase + r * rb) % 16
+                        if col * 16 < pre + seg:
+                            assert c * 16 + 16 <= tile - 16
+                            seen[r] = seen.get(r, 0) + 1
+                            assert c * 16 == r * ss + col * 16
+                    assert seen == {r: ((phase + r * rb) % 16 + seg + 15) // 16 for r in range(nr)}
+                    # a row's bytes in its LDS row, its last 32-bit read inside the tile
+                    assert all((phase + r * rb) % 16 + seg <= ss for r in range(nr))
+                    assert (nr - 1) * ss + (phase + (nr - 1) * rb) % 16 + seg + 7 <= tile
 
 
 @pytest.mark.parametrize("pre", [0, 2, 4, 6, 8, 10, 12, 14])
