@@ -331,18 +331,22 @@ def test_multi_token_on_matrix_cores(dev, t, nrows, ncols, ntok, off):
     assert (host(y).view(np.uint32) == np.asarray(yo).reshape(ntok, nrows).view(np.uint32)).all()
 
 
-@pytest.mark.parametrize("t", [O.IQ3_S, O.Q6_K, O.MXFP4])
-@pytest.mark.parametrize("nrows,ncols,ntok", [
-    (37, 256, 1), (16, 1280, 1), (50, 4352, 1), (33, 2816, 2), (35, 768, 4), (20, 4352, 8),
-])
-@pytest.mark.parametrize("off", [0, 2, 6])
+SUPER = [(37, 256, 1), (16, 1280, 1), (50, 4352, 1), (33, 2816, 2), (35, 768, 4), (20, 4352, 8)]
+BLOCKS = [(37, 96, 1), (35, 96, 4), (20, 2080, 4), (33, 2080, 7), (17, 4192, 8), (50, 4192, 1)]
+
+
+@pytest.mark.parametrize("t,nrows,ncols,ntok,off", [
+    (t, *s, off) for t in (O.IQ3_S, O.Q6_K, O.MXFP4) for s in SUPER for off in (0, 2, 6)
+] + [(O.MXFP4, *s, off) for s in BLOCKS for off in (0, 1, 7)     # 17-byte blocks: rows at odd bytes too
+] + [(t, *s, off) for t in (O.Q4_0, O.Q8_0) for s in BLOCKS for off in (0, 2)])
 def test_gemv_unaligned_rows(dev, t, nrows, ncols, ntok, off):
-    """Rows of an odd number of superblocks (each starts anywhere in a 16-byte
-    granule), whole and ragged chunks, matrices at any even address: bit-exact
-    against the oracle's (L=16, G=1) order."""
+    """Rows that start anywhere in a 16-byte granule (an odd number of
+    superblocks, or of 32-element blocks), whole and ragged chunks, matrices at
+    any even address (MXFP4: any): bit-exact against the oracle's (L=16, G=1)
+    order."""
     print(f"unaligned type={t} {nrows}x{ncols} ntok={ntok} off={off}", flush=True)
     rng = np.random.default_rng(nrows + ncols + ntok + t + off)
-    w = (O.quantize(t, rng.normal(0, 0.02, (nrows, ncols)).astype(np.float32)) if t == O.IQ3_S
+    w = (O.quantize(t, rng.normal(0, 0.02, (nrows, ncols)).astype(np.float32)) if t in (O.IQ3_S, O.Q4_0, O.Q8_0)
          else npref.rand_kq(t, nrows, ncols, rng))
     xq = O.quantize_q8_1(rng.standard_normal((ntok, ncols)).astype(np.float32))
     buf = torch.zeros(w.size + 32, dtype=torch.uint8, device=dev)

@@ -7,6 +7,9 @@ blocks in ascending order).  BASELINE config 5 (512 tokens, Q4_0, full
 shape) is checked token by token against the oracle for the whole chunk,
 plus chunk-independence and agreement with the decode entry point's
 routing."""
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -16,6 +19,15 @@ from chimere_amd.moe import MoeLayer
 from test_gpu_moe import build, check_margin, host, oracle_run, qmat
 
 pytestmark = pytest.mark.gpu
+
+
+def tile_pairs(E, K, T):
+    """Pairs per GEMM tile by the rule in the source (pf_tile_pairs, prefill.hip)."""
+    src = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "chimere_amd", "csrc", "prefill.hip")
+    with open(src) as f:
+        lo, hi = re.search(r"avg <= (\d+) \? PF_PT : avg <= (\d+) \? 2 \* PF_PT : 4 \* PF_PT", f.read()).groups()
+    avg = T * K / E
+    return 16 if avg <= int(lo) else 32 if avg <= int(hi) else 64
 
 
 def prefill_check(layer, x, sample=None, margin=True):
@@ -223,22 +235,49 @@ def test_prefill_model_layer_types_full_shape(dev):
 
 @pytest.mark.parametrize("et", [O.Q4_0, O.Q8_0, O.IQ3_S])
 @pytest.mark.parametrize("st", [None, O.Q4_0, O.Q8_0, O.IQ3_S, O.Q4_K, O.Q5_K, O.Q6_K])
-@pytest.mark.parametrize("H,F,E,K,T", [
-    (256, 256, 16, 1, 11),     # one K chunk; tiles of 16 pairs
-    (768, 512, 8, 2, 33),      # three gate/up chunks, two down chunks; tiles of 32, one of a single pair (shared)
-    (768, 256, 4, 2, 130),     # tiles of 64: full ones, short ones, one of 2 (shared)
+@pytest.mark.parametrize("H,F,E,K,T,tp", [
+    (256, 256, 16, 1, 11, 16),     # one K chunk
+    (768, 512, 8, 2, 65, 32),      # three gate/up chunks, two down chunks; 16.25 pairs per expert; shared tiles 32, 32, 1
+    (768, 256, 4, 2, 130, 64),     # full tiles, short ones, one of 2 (shared)
 ])
-def test_prefill_tile_sizes(dev, et, st, H, F, E, K, T):
+def test_prefill_tile_sizes(dev, et, st, H, F, E, K, T, tp):
     """Every expert x shared type at the three tile sizes (chosen by the
     average pairs per expert), odd and even numbers of K chunks, full and
     short tiles: bit-exact against the oracle's L=1 order."""
     print(f"prefill tiles et={et} st={st} H={H} F={F} E={E} K={K} T={T}", flush=True)
+    assert tile_pairs(E, K, T) == tp
     if st in (O.Q4_K, O.Q5_K, O.Q6_K):
         layer = kq_layer(dev, 900 + et + st + T, et, st, H, F, E, K)
     else:
         layer = build(dev, 900 + et + (st or 0) + T, H=H, F=F, E=E, K=K, et=et, st=st, gate_vec=st is not None)
     g = torch.Generator(device=dev).manual_seed(T + et)
     prefill_check(layer, torch.randn(T, H, generator=g, device=dev))
+
+
+def test_prefill_model_types_usual_chunk(dev):
+    """512 tokens of the model's layer types at its shape (IQ3_S experts, Q5_K
+    shared expert; tiles of 32 pairs): sampled tokens bit-exact against the
+    oracle, finite everywhere, every expert used."""
+    print("prefill IQ3_S + Q5_K shared, full shape, 512 tokens", flush=True)
+    assert tile_pairs(256, 8, 512) == 32
+    layer = kq_layer(dev, 881, O.IQ3_S, O.Q5_K, 2048, 512, 256, 8)
+    g = torch.Generator(device=dev).manual_seed(87)
+    og, ig, _ = prefill_check(layer, torch.randn(512, 2048, generator=g, device=dev), sample=list(range(0, 512, 11)))
+    assert np.isfinite(og).all()
+    assert (np.bincount(ig.reshape(-1), minlength=256) > 0).all()
+
+
+@pytest.mark.parametrize("E,K,T", [
+    (300, 12, 70),      # over 256 experts: two threads sum each one's counts
+    (257, 16, 16),      # one top-k work-group, all 256 of its pair threads
+    (1024, 16, 65),     # the most experts and pairs: a full plan work-group and one token more
+])
+def test_prefill_plan_many_experts(dev, E, K, T):
+    """The plan's branches for more than 256 experts and 16 pairs per token."""
+    print(f"prefill plan E={E} K={K} T={T}", flush=True)
+    layer = build(dev, 970 + E, H=256, F=256, E=E, K=K)
+    g = torch.Generator(device=dev).manual_seed(E + T)
+    prefill_check(layer, torch.randn(T, 256, generator=g, device=dev))
 
 
 @pytest.mark.parametrize("et", [O.Q4_0, O.Q8_0, O.IQ3_S])
@@ -273,3 +312,25 @@ def test_prefill_subnormal_activations(dev):
     for i, s in enumerate((1e-38, 1e-41, 1e-43, 3e-45, 1e-6)):
         x[3 * i] *= s
     prefill_check(layer, x, margin=False)
+
+
+@pytest.mark.parametrize("st", [O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("T", [20, 65, 130])
+def test_prefill_kquant_shared_offsets(dev, st, T):
+    """K-quant shared tensors at any even address (16-, 32- and 64-pair tiles) give
+    the bits of aligned ones."""
+    print(f"prefill shared offsets st={st} T={T}", flush=True)
+    layer = kq_layer(dev, 990 + st, O.IQ3_S, st, 512, 512, 8, 2)
+    g = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn(T, 512, generator=g, device=dev)
+    want = host(layer.prefill(x))
+    for off in (2, 6, 12):
+        moved = []
+        for k, t in enumerate(layer.tensors[6:9]):
+            buf = torch.zeros(t.numel() + 32, dtype=torch.uint8, device=dev)
+            o = (off + 2 * k) % 16
+            buf[o:o + t.numel()] = t.reshape(-1)
+            moved.append(buf[o:o + t.numel()])
+        other = MoeLayer(*layer.tensors[:4], O.IQ3_S, 2, shared=tuple(moved), shared_type=st,
+                         sh_gate_w=layer.tensors[4])
+        assert (host(other.prefill(x)).view(np.uint32) == want.view(np.uint32)).all()
