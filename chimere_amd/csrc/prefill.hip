@@ -242,8 +242,9 @@ __global__ __launch_bounds__(1024) void k_pf_plan(PfArgs a) {
     const int p0 = blockIdx.x * PF_PLG * PF_TKT * a.K, np = min(TK - p0, PF_PLG * PF_TKT * a.K);
     const int e = tid < np ? a.ids[p0 + tid] : -1;
     const int rank = tid < np ? a.rank[p0 + tid] : 0;
-    if (blockIdx.x == 0)
-        for (int i = tid; i < a.tile_slots; i += 1024) a.tiles[i] = make_int4(0, 0, 0, 0);
+    if (blockIdx.x == 0 && a.whole)
+        for (int i = tid; i < 8 * (pf_eighth(a.nsh) + pf_eighth(a.max_tiles)); i += 1024)
+            a.tiles[i] = make_int4(0, 0, 0, 0);
     total[tid] = 0;
     before[tid] = 0;
     __syncthreads();
@@ -286,25 +287,22 @@ __global__ __launch_bounds__(1024) void k_pf_plan(PfArgs a) {
         a.stok[tot[0] + t0 + tid] = t0 + tid;
     }
     if (blockIdx.x != 0) return;
-    // tile -> slot 8 g + x of XCD x: the shared expert's tiles (full ones, and
-    // of the slower types) come first, dealt one by one; then XCD x has a
-    // contiguous eighth of the experts' tiles (those of one expert share its
-    // weights in that L2).  With the shared tiles last in one contiguous split
-    // one XCD had them all: 4096 tokens IQ3_S + Q5_K gate/up 774 against 562 us.
-    const int n0 = (c0 + TP - 1) / TP, n1 = (c1 + TP - 1) / TP;
+    // the tile list, arranged for pf_place
+    const int n0 = (c0 + TP - 1) / TP, n1 = (c1 + TP - 1) / TP, nsh = a.nsh;
     const int to = excl_scan1024(n0 + n1, wsum, &tot[1]);
-    __syncthreads();
-    const int nsh = a.has_shared ? (a.T + TP - 1) / TP : 0, ne = tot[1];
-    const int per = max((ne + 7) >> 3, 1), persh = (nsh + 7) >> 3;
+    const int per = max(pf_eighth(tot[1]), 1), persh = pf_eighth(nsh);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const int c = h ? c1 : c0, base = h ? po + c0 : po, tb = h ? to + n0 : to;
         for (int s = 0; s * TP < c; s++) {
             const int t = tb + s, x = t / per;
-            a.tiles[8 * (persh + t - x * per) + x] = make_int4(2 * tid + h, base + s * TP, min(TP, c - s * TP), 0);
+            a.tiles[a.whole ? 8 * (persh + t - x * per) + x : 1 + nsh + t] =
+                make_int4(2 * tid + h, base + s * TP, min(TP, c - s * TP), 0);
         }
     }
-    for (int s = tid; s < nsh; s += 1024) a.tiles[s] = make_int4(E, tot[0] + s * TP, min(TP, a.T - s * TP), 0);
+    for (int s = tid; s < nsh; s += 1024)
+        a.tiles[a.whole ? s : 1 + s] = make_int4(E, tot[0] + s * TP, min(TP, a.T - s * TP), 0);
+    if (tid == 0 && !a.whole) a.tiles[0] = make_int4(tot[1], 0, 0, 0);
 }
 
 // P6: grid (ceil(H/256), T): out = sum_k fmaf(w_k, dn_k, acc) (+ shared expert)
@@ -351,7 +349,7 @@ __global__ __launch_bounds__(256) void k_pf_combine(PfArgs a) {
 
 struct PfPlan {
     size_t logits, glogit, ids, wts, cnt, rank, spairs, stok, tiles, dn, xh, xd, xs, hh, hd, hs, total;
-    int tile_slots, tile_pairs;
+    int tile_pairs, nsh, max_tiles, whole;
 };
 
 static size_t al256p(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -369,15 +367,21 @@ static int pf_tile_pairs(int E, int K, int T) {
     return avg <= 13 ? PF_PT : avg <= 20 ? 2 * PF_PT : 4 * PF_PT;
 }
 
+// The experts' tiles (at most) above which whole tiles are dealt to the XCDs
+// (both sides measured at pf_place: slices are faster up to 343 tiles, even at
+// 381, slower at 768; by whole tiles an XCD has at most 12 / tiles more than the average)
+constexpr int PF_WHOLE_TILES = 512;
+
 static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     PfPlan p{};
     size_t o = 0;
     const size_t P = (size_t)T * K + T;
     p.tile_pairs = pf_tile_pairs(E, K, T);
-    // tiles: at most P / tile_pairs + E + 1; the experts' and the shared ones
-    // are rounded up to whole rounds of 8 apart
-    auto slots = [&](int tp) { return ((int)(P / tp) + E + 1 + 14 + 7) / 8 * 8; };
-    p.tile_slots = slots(p.tile_pairs);
+    // an expert of c pairs has at most c / tile_pairs + 1 tiles
+    auto tiles = [&](int tp) { return T * K / tp + (T * K < E ? T * K : E); };
+    p.max_tiles = tiles(p.tile_pairs);
+    p.nsh = (T + p.tile_pairs - 1) / p.tile_pairs;
+    p.whole = p.max_tiles > PF_WHOLE_TILES;
     auto take = [&](size_t& at, size_t bytes) { at = o; o += al256p(bytes); };
     take(p.logits, (size_t)T * E * 4);
     take(p.glogit, (size_t)T * 4);
@@ -387,7 +391,7 @@ static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     take(p.rank, (size_t)T * K * 4);
     take(p.spairs, P * 4);
     take(p.stok, P * 4);
-    take(p.tiles, (size_t)slots(PF_PT) * sizeof(int4));
+    take(p.tiles, (size_t)(tiles(PF_PT) + (T + PF_PT - 1) / PF_PT + 16) * sizeof(int4));
     take(p.dn, P * H * 4);
     take(p.xh, (size_t)T * H * 2);
     take(p.xd, (size_t)T * (H / QK) * 4);
@@ -471,7 +475,7 @@ void chimere_moe_prefill(const chimere_moe_layer* L, const float* x, float* out,
     a.dn = (float*)(w + p.dn);
     a.xh = (_Float16*)(w + p.xh); a.xd = (uint32_t*)(w + p.xd); a.xs = (float*)(w + p.xs);
     a.hh = (_Float16*)(w + p.hh); a.hd = (uint32_t*)(w + p.hd); a.hs = (float*)(w + p.hs);
-    a.tile_slots = p.tile_slots; a.tile_pairs = p.tile_pairs;
+    a.tile_pairs = p.tile_pairs; a.nsh = has_sh ? p.nsh : 0; a.max_tiles = p.max_tiles; a.whole = p.whole;
     launch_pf(a, L->expert_type, has_sh ? L->shared_type : L->expert_type, stream);
     check_launch("moe_prefill");
 }

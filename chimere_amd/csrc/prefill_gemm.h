@@ -54,7 +54,7 @@ struct PfArgs {
     int* rank;       // [T*K] a pair's place among its expert's of its top-k work-group
     int* spairs;     // [T*K + T] pairs grouped by expert (shared expert last)
     int* stok;       // [T*K + T] the pairs' tokens, in the same order
-    int4* tiles;     // [tile_slots] (expert, first position in spairs, pairs or 0)
+    int4* tiles;     // (expert, first position in spairs, pairs or 0) of each tile, arranged for pf_place
     float* dn;       // [T*K + T][H] down-projection output per pair
     // Q8_1 blocks of x (by token) and of h (by position in spairs) as the
     // GEMMs read them: the quants as f16, the block's f16 scale in the low
@@ -63,8 +63,10 @@ struct PfArgs {
     _Float16 *xh, *hh;
     uint32_t *xd, *hd;
     float *xs, *hs;
-    int tile_slots;   // a multiple of 8
     int tile_pairs;   // most pairs per tile: PF_PT * MT of the GEMM launches
+    int nsh;          // tiles of the shared expert
+    int max_tiles;    // most tiles of the experts
+    int whole;        // whole tiles are dealt to the XCDs (pf_place)
 };
 
 // ---- a weight row's chunk in LDS
@@ -581,14 +583,45 @@ constexpr int pf_xb() { return pf_ch<T>() == 8 && M == 2 && !ONE ? 8 : 4; }
 template <int MT, bool ONE>
 constexpr int pf_xu() { return MT == 2 && !ONE ? 16 : 4 * MT; }
 
-// Work-group -> (slot of the tile list, slice of rows).  The hardware deals
-// work-groups to the 8 XCDs round-robin; slots 8 g + x are XCD x's, and the
-// row slices of one tile follow each other on one XCD: the tile's activation
-// rows are fetched into that L2 once.
+// Work-group -> (tile, slice of rows); pairs 0: none.  The hardware deals
+// work-groups to the 8 XCDs round-robin, and the slices of one tile follow each
+// other on one XCD: its activation rows are fetched into that L2 once, and
+// the tiles of one expert (consecutive) share its weights there.  The shared
+// expert's tiles (full ones, and of the slower types) are dealt apart from the
+// experts' and come first: with them at the end of one list a single XCD had
+// them all, 4096 tokens IQ3_S + Q5_K gate/up 774 against 562 us.
+//  * whole tiles: entry 8 g + x is XCD x's g-th, the shared expert's dealt one
+//    by one, the experts' in contiguous eighths, pairs 0 in unused entries;
+//  * otherwise XCD x has a contiguous eighth of each part's (tile, slice) list:
+//    entry 0 has the number of the experts' tiles, then follow the shared
+//    expert's and the experts'.  Few tiles are bound by each XCD's weight
+//    stream, and by whole tiles an XCD had up to two more than another (35
+//    tiles: 6 and none; halves of tiles: still 13 % more than the average).
+// Whole tiles / slices (us): 12 tokens, H = 4096, F = 1024, 64 experts, top-4
+// Q8_0 144 / 112, IQ3_S + Q5_K 117 / 95; H = 2048, F = 512, 256 experts, top-8:
+// 9 tokens Q8_0 77 / 64, IQ3_S + Q5_K 72 / 62; 700 tokens IQ3_S + Q5_K 248 / 243;
+// 1000 tokens 305 / 306, Q8_0 336 / 332, Q4_0 283 / 285; 4096 tokens (about 700
+// tiles; the count is one more load that a tile's waits for) 808 / 822, Q4_0 733 / 747.
+__host__ __device__ constexpr int pf_eighth(int n) { return (n + 7) >> 3; }
 __device__ __forceinline__ int4 pf_place(const PfArgs& a, int nslice, int& sl) {   // nslice: work-groups per tile
-    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, g = k / nslice;
-    sl = k - g * nslice;
-    return a.tiles[8 * g + x];
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
+    if (a.whole) {
+        const int g = k / nslice;
+        sl = k - g * nslice;
+        return a.tiles[8 * g + x];
+    }
+    const int ps = pf_eighth(a.nsh * nslice);
+    const bool sh = k < ps;
+    const int n = (sh ? a.nsh : a.tiles[0].x) * nslice, per = pf_eighth(n), i = sh ? k : k - ps;
+    const int w = x * per + i, t = w / nslice;
+    sl = w - t * nslice;
+    if (i >= per || w >= n) return make_int4(0, 0, 0, 0);
+    return a.tiles[1 + (sh ? 0 : a.nsh) + t];
+}
+// work-groups of a launch
+inline int pf_grid(const PfArgs& a, int nslice) {
+    if (a.whole) return 8 * (pf_eighth(a.nsh) + pf_eighth(a.max_tiles)) * nslice;
+    return 8 * (pf_eighth(a.nsh * nslice) + pf_eighth(a.max_tiles * nslice));
 }
 
 // LDS arrays of a work-group
@@ -756,8 +789,8 @@ __global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, true>() ? 3 : 2)) vo
 
 template <int TE, int TS, int MT>
 void pf_launch_mt(const PfArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL((k_pf_gate_up<TE, TS, MT>), dim3(a.F / 64 * a.tile_slots), dim3(PF_THREADS), 0, s, a);
-    hipLaunchKernelGGL((k_pf_down<TE, TS, MT>), dim3(a.H / (PF_ROWS * PF_DN_NS) * a.tile_slots), dim3(PF_THREADS), 0, s, a);
+    hipLaunchKernelGGL((k_pf_gate_up<TE, TS, MT>), dim3(pf_grid(a, a.F / 64)), dim3(PF_THREADS), 0, s, a);
+    hipLaunchKernelGGL((k_pf_down<TE, TS, MT>), dim3(pf_grid(a, a.H / (PF_ROWS * PF_DN_NS))), dim3(PF_THREADS), 0, s, a);
 }
 
 // gate/up and down launches of one expert type, a.tile_pairs = 16 * MT pairs per tile

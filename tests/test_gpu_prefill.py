@@ -280,6 +280,19 @@ def test_prefill_plan_many_experts(dev, E, K, T):
     prefill_check(layer, torch.randn(T, 256, generator=g, device=dev))
 
 
+@pytest.mark.parametrize("H,K,st", [(256, 8, O.Q4_0), (1024, 8, O.Q8_0), (256, 8, None)])
+def test_prefill_whole_tile_dealing(dev, H, K, st):
+    """4000 tokens (more tiles than the rule's line: whole tiles go to the XCDs)
+    have the bits of chunks of 100 and, sampled, of the oracle."""
+    print(f"prefill whole tiles H={H} K={K} st={st}", flush=True)
+    layer = build(dev, 1010 + H, H=H, F=256, E=64, K=K, st=st)
+    g = torch.Generator(device=dev).manual_seed(H)
+    x = torch.randn(4000, H, generator=g, device=dev)
+    og, _, _ = prefill_check(layer, x, sample=list(range(7, 4000, 400)))
+    for t in range(0, 4000, 100):
+        assert (host(layer.prefill(x[t:t + 100])).view(np.uint32) == og[t:t + 100].view(np.uint32)).all(), t
+
+
 @pytest.mark.parametrize("et", [O.Q4_0, O.Q8_0, O.IQ3_S])
 @pytest.mark.parametrize("off", [2, 4, 14])
 def test_prefill_weight_offsets(dev, et, off):

@@ -227,31 +227,61 @@ def test_prefill_activation_stage(mt, xb):
                         (16 * (q % mt) + c, b + q // mt)
 
 
+def eighth(n):
+    return (n + 7) >> 3
+
+
+def pf_place(block, nslice, nsh, ne, whole):
+    """(tile, slice) of a work-group, shared tiles before the experts'; None: no work."""
+    x, k = block & 7, block >> 3
+    if whole:
+        g, sl = divmod(k, nslice)
+        per, persh = max(eighth(ne), 1), eighth(nsh)
+        slots = {s: s for s in range(nsh)}
+        slots.update({8 * (persh + t - t // per * per) + t // per: nsh + t for t in range(ne)})
+        t = slots.get(8 * g + x)
+        return None if t is None else (t, sl)
+    ps = eighth(nsh * nslice)
+    n, i = (nsh * nslice, k) if k < ps else (ne * nslice, k - ps)
+    w = x * eighth(n) + i
+    return None if i >= eighth(n) or w >= n else (w // nslice + (0 if k < ps else nsh), w % nslice)
+
+
 @pytest.mark.parametrize("tp", [16, 32, 64])
-@pytest.mark.parametrize("E,K,T", [(1, 1, 1), (4, 2, 33), (8, 8, 130), (256, 8, 45), (256, 8, 512), (300, 12, 70),
+@pytest.mark.parametrize("E,K,T", [(1, 1, 1), (4, 2, 33), (8, 8, 130), (64, 4, 12), (256, 8, 9), (300, 12, 70),
                                    (1024, 16, 65)])
-def test_prefill_tile_slots(tp, E, K, T):
-    """The plan's tiles (experts' in contiguous eighths, one per XCD, after the
-    shared expert's) have a slot each inside the list, however the router deals
-    the pairs."""
+def test_prefill_tile_dealing(tp, E, K, T):
+    """However the router deals the pairs, the plan's tiles fit their list, every
+    slice of every tile belongs to one work-group of the launch, and (but for
+    whole tiles) no XCD has more than an eighth, rounded up, of either part's."""
     import random
     rng = random.Random(E * K + T)
-    slots = lambda n: ((T * K + T) // n + E + 1 + 14 + 7) // 8 * 8  # noqa: E731
-    assert slots(tp) <= slots(16)                               # the workspace's size
-    for shared in (False, True):
-        for case in range(8):
+    tiles = lambda n: T * K // n + min(T * K, E)  # noqa: E731
+    entries = tiles(16) + (T + 15) // 16 + 16                   # of the workspace
+    for shared, nslice in ((False, 4), (True, 16), (True, 1), (True, 3)):
+        for case in range(3):
             counts = [0] * E
             for _ in range(T):
-                hot = range(K) if case == 0 else sorted(rng.sample(range(E), K))
-                for e in hot:
+                for e in (range(K) if case == 0 else rng.sample(range(E), K)):
                     counts[e] += 1
             if case == 1:                                       # one pair left over everywhere it can be
                 counts = [tp + 1 if i < T * K // (tp + 1) else 0 for i in range(E)]
             ne = sum((c + tp - 1) // tp for c in counts)
             nsh = (T + tp - 1) // tp if shared else 0
-            per, persh = max((ne + 7) >> 3, 1), (nsh + 7) >> 3
-            used = list(range(nsh)) + [8 * (persh + t - t // per * per) + t // per for t in range(ne)]
-            assert len(set(used)) == ne + nsh and max(used, default=0) < slots(tp)
+            assert ne <= tiles(tp)
+            assert 1 + nsh + ne <= entries and 8 * (eighth(nsh) + eighth(tiles(tp))) <= entries
+            want = sorted((t, s) for t in range(nsh + ne) for s in range(nslice))
+            for whole in (False, True):
+                grid = (8 * (eighth(nsh) + eighth(tiles(tp))) * nslice if whole else
+                        8 * (eighth(nsh * nslice) + eighth(tiles(tp) * nslice)))
+                if grid > 20000:
+                    continue
+                got = [(b & 7, pf_place(b, nslice, nsh, ne, whole)) for b in range(grid)]
+                assert sorted(p for _, p in got if p) == want
+                if not whole:
+                    for part in (lambda t: t < nsh, lambda t: t >= nsh):
+                        load = [sum(1 for x, p in got if p and x == k and part(p[0])) for k in range(8)]
+                        assert max(load) == eighth(sum(load)) and load == sorted(load, reverse=True)
 
 
 @pytest.mark.parametrize("t", ["iq3s", "q6k", "mxfp4"])
