@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void k_pf_combine(PfArgs a) {
 
 struct PfPlan {
     size_t logits, glogit, ids, wts, cnt, rank, spairs, stok, tiles, dn, xh, xd, xs, hh, hd, hs, total;
-    int tile_pairs, nsh, max_tiles, whole;
+    int tile_pairs, nsh, max_tiles, whole, dn_ns;
 };
 
 static size_t al256p(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -371,6 +371,15 @@ static int pf_tile_pairs(int E, int K, int T) {
 // (both sides measured at pf_place: slices are faster up to 343 tiles, even at
 // 381, slower at 768; by whole tiles an XCD has at most 12 / tiles more than the average)
 constexpr int PF_WHOLE_TILES = 512;
+// Work-groups that the down launch would have at most (the tiles' bound) with two
+// slices each, up to which it takes one: two leave CUs idle behind the longest
+// chain of slices.  Chunk with two / one (us): H = F = 1024, 32 experts, top-2,
+// 12 tokens (104) IQ3_S + Q5_K 53 / 44, Q8_0 49 / 42, 1000 tokens (188) IQ3_S + Q5_K
+// 129 / 109; H = 4096, F = 1024, 64 experts, top-4, 100 tokens (1536) Q8_0 238 / 232,
+// 200 tokens (2032) 273 / 268; H = 2048, F = 512, 256 experts, top-8, 16 tokens
+// (1096) 110 / 107, 64 tokens (2336) Q8_0 187 / 185 but IQ3_S + Q5_K 132 / 134,
+// 512 tokens (3200) 212 / 216, Q4_0 195 / 199.
+constexpr int PF_DN_ONE = 2048;
 
 static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     PfPlan p{};
@@ -382,6 +391,7 @@ static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     p.max_tiles = tiles(p.tile_pairs);
     p.nsh = (T + p.tile_pairs - 1) / p.tile_pairs;
     p.whole = p.max_tiles > PF_WHOLE_TILES;
+    p.dn_ns = (int64_t)(p.max_tiles + p.nsh) * (H / (2 * PF_ROWS)) <= PF_DN_ONE ? 1 : 2;
     auto take = [&](size_t& at, size_t bytes) { at = o; o += al256p(bytes); };
     take(p.logits, (size_t)T * E * 4);
     take(p.glogit, (size_t)T * 4);
@@ -476,6 +486,7 @@ void chimere_moe_prefill(const chimere_moe_layer* L, const float* x, float* out,
     a.xh = (_Float16*)(w + p.xh); a.xd = (uint32_t*)(w + p.xd); a.xs = (float*)(w + p.xs);
     a.hh = (_Float16*)(w + p.hh); a.hd = (uint32_t*)(w + p.hd); a.hs = (float*)(w + p.hs);
     a.tile_pairs = p.tile_pairs; a.nsh = has_sh ? p.nsh : 0; a.max_tiles = p.max_tiles; a.whole = p.whole;
+    a.dn_ns = p.dn_ns;
     launch_pf(a, L->expert_type, has_sh ? L->shared_type : L->expert_type, stream);
     check_launch("moe_prefill");
 }

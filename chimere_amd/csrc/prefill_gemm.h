@@ -67,6 +67,7 @@ struct PfArgs {
     int nsh;          // tiles of the shared expert
     int max_tiles;    // most tiles of the experts
     int whole;        // whole tiles are dealt to the XCDs (pf_place)
+    int dn_ns;        // 128-row slices per work-group of the down launch: 1 or 2
 };
 
 // ---- a weight row's chunk in LDS
@@ -659,7 +660,7 @@ __device__ __forceinline__ void pf_dispatch(const int4& ti, bool sh, Run run) {
     else if constexpr (TE != TS) with(std::integral_constant<int, TS>{});
 }
 
-// P4: grid tile_slots * F / 64 work-groups: h = silu(gate) * up of 64 rows of
+// P4: F / 64 work-groups per tile (pf_place): h = silu(gate) * up of 64 rows of
 // F for a tile's pairs, as Q8_1 blocks (by position in spairs).  (Two and four
 // slices of rows per work-group, the next one's copies in flight during this
 // epilogue, measured slower: 512 tokens Q4_0 108 -> 118 and 144 us -- fewer
@@ -746,20 +747,19 @@ __global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, false>() ? 3 : 2)) v
     });
 }
 
-// P5: grid tile_slots * H / (128 PF_DN_NS) work-groups: slices of 128 down rows
+// P5: H / (128 dn_ns) work-groups per tile (pf_place): slices of 128 down rows
 // of a tile's pairs, K = F, by pair id.  K is short (16 blocks at F = 512), so
-// a work-group takes two slices and starts the second's copies before it
-// stores the first's outputs: 4096 tokens IQ3_S 248 -> 241 us, 1777 tokens
-// Q8_0 130 -> 121 us.
-constexpr int PF_DN_NS = 2;
+// a work-group of a large launch takes two slices and starts the second's copies
+// before it stores the first's outputs: 4096 tokens IQ3_S 248 -> 241 us, 1777
+// tokens Q8_0 130 -> 121 us.
 template <int TE, int TS, int MT>
 __global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, true>() ? 3 : 2)) void k_pf_down(PfArgs a) {
     constexpr bool ONE = pf_single<TS, MT, true>();
     int sl;
-    const int4 ti = pf_place(a, a.H / (PF_ROWS * PF_DN_NS), sl);
+    const int4 ti = pf_place(a, a.H / (PF_ROWS * a.dn_ns), sl);
     if (ti.z == 0) return;
     PF_LDS_ARRAYS;
-    const int e = ti.x, r0 = sl * PF_DN_NS * PF_ROWS;
+    const int e = ti.x, r0 = sl * a.dn_ns * PF_ROWS;
     const bool sh = e == a.E;
     const uint8_t* d = sh ? a.sh_down : a.down + (int64_t)e * a.sd;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c = lane & 15;
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, true>() ? 3 : 2)) vo
         for (int m = 0; m < M; m++)
 #pragma unroll
             for (int i = 0; i < 4; i++) prs[m][i] = a.spairs[start + min(16 * m + 4 * q + i, np - 1)];
-        pf_gemm<T, M, pf_xb<T, M, ONE>(), pf_wdb<T, TE, TS, ONE>()>(L, d + r0 * rb, d + (r0 + 64) * rb, rb, PF_DN_NS, PF_ROWS * rb, a.F / QK,
+        pf_gemm<T, M, pf_xb<T, M, ONE>(), pf_wdb<T, TE, TS, ONE>()>(L, d + r0 * rb, d + (r0 + 64) * rb, rb, a.dn_ns, PF_ROWS * rb, a.F / QK,
                                            a.hh, a.hd, a.hs, nullptr, start, np, grid, [&](int s, float (&acc)[2][M][4]) {
             const int r = r0 + s * PF_ROWS + 16 * wave + c;
 #pragma unroll
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(PF_THREADS, (pf_single<TS, MT, true>() ? 3 : 2)) vo
 template <int TE, int TS, int MT>
 void pf_launch_mt(const PfArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_pf_gate_up<TE, TS, MT>), dim3(pf_grid(a, a.F / 64)), dim3(PF_THREADS), 0, s, a);
-    hipLaunchKernelGGL((k_pf_down<TE, TS, MT>), dim3(pf_grid(a, a.H / (PF_ROWS * PF_DN_NS))), dim3(PF_THREADS), 0, s, a);
+    hipLaunchKernelGGL((k_pf_down<TE, TS, MT>), dim3(pf_grid(a, a.H / (PF_ROWS * a.dn_ns))), dim3(PF_THREADS), 0, s, a);
 }
 
 // gate/up and down launches of one expert type, a.tile_pairs = 16 * MT pairs per tile
