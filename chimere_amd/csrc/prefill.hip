@@ -368,9 +368,12 @@ static int pf_tile_pairs(int E, int K, int T) {
 }
 
 // The experts' tiles (at most) above which whole tiles are dealt to the XCDs
-// (both sides measured at pf_place: slices are faster up to 343 tiles, even at
-// 381, slower at 768; by whole tiles an XCD has at most 12 / tiles more than the average)
-constexpr int PF_WHOLE_TILES = 512;
+// (by whole tiles an XCD has at most 12 / tiles more than the average).  Whole /
+// slices (us), H = 2048, F = 512, 256 experts, top-8: 343 tiles IQ3_S + Q5_K 248 / 243;
+// 384 Q4_0 193.1 / 193.6; 408 Q4_0 + Q6_K 235 / 223, IQ3_S + Q5_K 239 / 228, Q4_0
+// 205 / 209; 464 IQ3_S + Q5_K 216 / 218, Q4_0 186 / 189, Q4_0 + Q6_K 195 / 199; 768
+// IQ3_S + Q5_K 808 / 822, Q4_0 733 / 747
+constexpr int PF_WHOLE_TILES = 432;
 // Work-groups that the down launch would have at most (the tiles' bound) with two
 // slices each, up to which it takes one: two leave CUs idle behind the longest
 // chain of slices.  Chunk with two / one (us): H = F = 1024, 32 experts, top-2,

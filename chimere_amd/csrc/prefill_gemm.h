@@ -600,9 +600,8 @@ constexpr int pf_xu() { return MT == 2 && !ONE ? 16 : 4 * MT; }
 //    tiles: 6 and none; halves of tiles: still 13 % more than the average).
 // Whole tiles / slices (us): 12 tokens, H = 4096, F = 1024, 64 experts, top-4
 // Q8_0 144 / 112, IQ3_S + Q5_K 117 / 95; H = 2048, F = 512, 256 experts, top-8:
-// 9 tokens Q8_0 77 / 64, IQ3_S + Q5_K 72 / 62; 700 tokens IQ3_S + Q5_K 248 / 243;
-// 1000 tokens 305 / 306, Q8_0 336 / 332, Q4_0 283 / 285; 4096 tokens (about 700
-// tiles; the count is one more load that a tile's waits for) 808 / 822, Q4_0 733 / 747.
+// 9 tokens Q8_0 77 / 64, IQ3_S + Q5_K 72 / 62.  Many tiles are even enough whole,
+// without the load of the count that the tile's waits for (PF_WHOLE_TILES).
 __host__ __device__ constexpr int pf_eighth(int n) { return (n + 7) >> 3; }
 __device__ __forceinline__ int4 pf_place(const PfArgs& a, int nslice, int& sl) {   // nslice: work-groups per tile
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
