@@ -381,8 +381,10 @@ constexpr int PF_WHOLE_TILES = 432;
 // 129 / 109; H = 4096, F = 1024, 64 experts, top-4, 100 tokens (1536) Q8_0 238 / 232,
 // 200 tokens (2032) 273 / 268; H = 2048, F = 512, 256 experts, top-8, 16 tokens
 // (1096) 110 / 107, 64 tokens (2336) Q8_0 187 / 185 but IQ3_S + Q5_K 132 / 134,
-// 512 tokens (3200) 212 / 216, Q4_0 195 / 199.
-constexpr int PF_DN_ONE = 2048;
+// 512 tokens (3200) 212 / 216, Q4_0 195 / 199.  Rows of one K chunk (F = 256) are all
+// start: H = 1024, 64 experts, top-6, 500 tokens (472) IQ3_S + Q5_K 70.5 / 66.3, Q8_0
+// 63.7 / 64.8, 1500 tokens (912) 110.7 / 111.7, 103.8 / 105.2.
+constexpr int PF_DN_ONE = 2048, PF_DN_ONE_K8 = 512;
 
 static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     PfPlan p{};
@@ -394,7 +396,7 @@ static PfPlan plan_pf(int H, int F, int E, int K, int T) {
     p.max_tiles = tiles(p.tile_pairs);
     p.nsh = (T + p.tile_pairs - 1) / p.tile_pairs;
     p.whole = p.max_tiles > PF_WHOLE_TILES;
-    p.dn_ns = (int64_t)(p.max_tiles + p.nsh) * (H / (2 * PF_ROWS)) <= PF_DN_ONE ? 1 : 2;
+    p.dn_ns = (int64_t)(p.max_tiles + p.nsh) * (H / (2 * PF_ROWS)) <= (F > 256 ? PF_DN_ONE : PF_DN_ONE_K8) ? 1 : 2;
     auto take = [&](size_t& at, size_t bytes) { at = o; o += al256p(bytes); };
     take(p.logits, (size_t)T * E * 4);
     take(p.glogit, (size_t)T * 4);
