@@ -357,14 +357,23 @@ static size_t al256p(size_t n) { return (n + 255) & ~(size_t)255; }
 // Pairs per GEMM tile, by the average pairs per expert: a weight block is
 // decoded once per tile, so a tile should hold an expert's pairs, but a wider
 // tile's LDS and registers leave two work-groups per CU instead of three.
-// H = 2048, F = 512, E = 256, top-8, 16 / 32 / 64 pairs: IQ3_S + Q5_K shared
-// 350 tokens (average 11) 186 / 202 / 217 us, 512 (16) 238 / 219 / 226, 800
-// (25) 321 / 271 / 265; Q4_0 350 173 / 185 / 196, 512 206 / 202 / 206, 800
-// 271 / 237 / 231; Q8_0 350 254 / 257 / 263, 512 297 / 274 / 276, 800 364 /
-// 306 / 305.
-static int pf_tile_pairs(int E, int K, int T) {
+// Of 32 pairs and 64, the wider tile decodes fewer blocks but has a short tile
+// per expert; it gains earlier with Q8_0 experts (more bytes per block).
+// Chunk, 16 / 32 / 64 pairs (us), H = 2048, F = 512, 256 experts, top-8, by average:
+//   IQ3_S + Q5_K  11 190 / 197 / 218   13 205 / 203 / 221   15 224 / 213 / 226
+//                 24 308 / 249 / 252   28 339 / 278 / 276   32 371 / 311 / 298
+//   Q4_0          11 174 / 180 / 198   13 185 / 183 / 203   24 267 / 228 / 229
+//                 28 291 / 248 / 250   32 318 / 274 / 269
+//   Q8_0          11 256 / 253 / 264   13 266 / 257 / 270   20 332 / 280 / 289
+//                 22 343 / 287 / 293   24 358 / 309 / 300   28 386 / 330 / 314
+// H = F = 1024, 64 experts, top-4: IQ3_S + Q5_K 13 76 / 79 / 92, 17 93 / 89 / 95, 28
+// 115 / 98 / 104; H = 2048, F = 768, 16 experts, top-2: 20 65 / 73 / 86, 40 94 / 86 / 89.
+// Skewed (logits lowered by the log of the expert's rank), IQ3_S + Q5_K: 8 138 / 123 /
+// 137, 13 187 / 157 / 178, 20 249 / 207 / 215, 35 395 / 313 / 311: the average understates
+// the experts that most pairs meet (Q8_0 20 290 / 232 / 218).
+static int pf_tile_pairs(int te, int E, int K, int T) {
     const double avg = (double)T * K / E;
-    return avg <= 13 ? PF_PT : avg <= 20 ? 2 * PF_PT : 4 * PF_PT;
+    return avg <= 13 ? PF_PT : avg <= (te == T_Q8_0 ? 20 : 28) ? 2 * PF_PT : 4 * PF_PT;
 }
 
 // The experts' tiles (at most) above which whole tiles are dealt to the XCDs
@@ -386,11 +395,11 @@ constexpr int PF_WHOLE_TILES = 432;
 // 63.7 / 64.8, 1500 tokens (912) 110.7 / 111.7, 103.8 / 105.2.
 constexpr int PF_DN_ONE = 2048, PF_DN_ONE_K8 = 512;
 
-static PfPlan plan_pf(int H, int F, int E, int K, int T) {
+static PfPlan plan_pf(int te, int H, int F, int E, int K, int T) {
     PfPlan p{};
     size_t o = 0;
     const size_t P = (size_t)T * K + T;
-    p.tile_pairs = pf_tile_pairs(E, K, T);
+    p.tile_pairs = pf_tile_pairs(te, E, K, T);
     // an expert of c pairs has at most c / tile_pairs + 1 tiles
     auto tiles = [&](int tp) { return T * K / tp + (T * K < E ? T * K : E); };
     p.max_tiles = tiles(p.tile_pairs);
@@ -439,7 +448,7 @@ extern "C" {
 
 size_t chimere_moe_prefill_workspace_size(const chimere_moe_layer* L, int max_ntok) {
     if (!L || max_ntok < 1) return 0;
-    return plan_pf(L->hidden, L->ffn, L->n_experts, L->top_k, max_ntok).total;
+    return plan_pf(L->expert_type, L->hidden, L->ffn, L->n_experts, L->top_k, max_ntok).total;
 }
 
 void chimere_moe_prefill(const chimere_moe_layer* L, const float* x, float* out, int ntok, int* ids_out,
@@ -470,7 +479,7 @@ void chimere_moe_prefill(const chimere_moe_layer* L, const float* x, float* out,
     CHIMERE_REQUIRE((((uintptr_t)L->gate_exps | (uintptr_t)L->up_exps | (uintptr_t)L->down_exps |
                       (uintptr_t)L->gate_stride | (uintptr_t)L->up_stride | (uintptr_t)L->down_stride) & 1) == 0,
                     CHIMERE_ERR_ARG, "moe_prefill: weights must be 2-byte aligned");
-    const PfPlan p = plan_pf(H, F, E, K, ntok);
+    const PfPlan p = plan_pf(L->expert_type, H, F, E, K, ntok);
     CHIMERE_REQUIRE(ws_bytes >= p.total && ((uintptr_t)workspace & 255) == 0, CHIMERE_ERR_WORKSPACE,
                     "moe_prefill: workspace %zu bytes < %zu (or not 256-byte aligned)", ws_bytes, p.total);
     uint8_t* w = (uint8_t*)workspace;

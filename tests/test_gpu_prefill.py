@@ -21,13 +21,14 @@ from test_gpu_moe import build, check_margin, host, oracle_run, qmat
 pytestmark = pytest.mark.gpu
 
 
-def tile_pairs(E, K, T):
+def tile_pairs(et, E, K, T):
     """Pairs per GEMM tile by the rule in the source (pf_tile_pairs, prefill.hip)."""
     src = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "chimere_amd", "csrc", "prefill.hip")
     with open(src) as f:
-        lo, hi = re.search(r"avg <= (\d+) \? PF_PT : avg <= (\d+) \? 2 \* PF_PT : 4 \* PF_PT", f.read()).groups()
+        lo, *hi = re.search(r"avg <= (\d+) \? PF_PT : avg <= \(te == T_Q8_0 \? (\d+) : (\d+)\) \? 2 \* PF_PT : 4 \* PF_PT",
+                            f.read()).groups()
     avg = T * K / E
-    return 16 if avg <= int(lo) else 32 if avg <= int(hi) else 64
+    return 16 if avg <= int(lo) else 32 if avg <= int(hi[et != O.Q8_0]) else 64
 
 
 def prefill_check(layer, x, sample=None, margin=True):
@@ -245,7 +246,7 @@ def test_prefill_tile_sizes(dev, et, st, H, F, E, K, T, tp):
     average pairs per expert), odd and even numbers of K chunks, full and
     short tiles: bit-exact against the oracle's L=1 order."""
     print(f"prefill tiles et={et} st={st} H={H} F={F} E={E} K={K} T={T}", flush=True)
-    assert tile_pairs(E, K, T) == tp
+    assert tile_pairs(et, E, K, T) == tp
     if st in (O.Q4_K, O.Q5_K, O.Q6_K):
         layer = kq_layer(dev, 900 + et + st + T, et, st, H, F, E, K)
     else:
@@ -259,7 +260,7 @@ def test_prefill_model_types_usual_chunk(dev):
     shared expert; tiles of 32 pairs): sampled tokens bit-exact against the
     oracle, finite everywhere, every expert used."""
     print("prefill IQ3_S + Q5_K shared, full shape, 512 tokens", flush=True)
-    assert tile_pairs(256, 8, 512) == 32
+    assert tile_pairs(O.IQ3_S, 256, 8, 512) == 32
     layer = kq_layer(dev, 881, O.IQ3_S, O.Q5_K, 2048, 512, 256, 8)
     g = torch.Generator(device=dev).manual_seed(87)
     og, ig, _ = prefill_check(layer, torch.randn(512, 2048, generator=g, device=dev), sample=list(range(0, 512, 11)))
