@@ -410,12 +410,12 @@ def main():
         tp, _ = graph_time(fns)
         upf = tp / 16
         pairs = T * K + T                                   # routed pairs + shared expert rows
-        ops = pairs * 2 * (2 * F * H + H * F)               # int8 MACs x2 of gate, up, down
+        ops = pairs * 2 * (2 * F * H + H * F)               # 2 per multiply-add of gate, up, down
         pbytes = (ue + 1) * expert_bytes + E * H * 4 + 2 * T * H * 4
         extra["prefill_q4_0_512"] = {
             "us_per_chunk": round(upf * 1e6, 2), "tokens_per_s": round(T / upf, 1), "unique_experts": ue,
             "GBs_unique_weight_bytes": round(pbytes / upf / 1e9, 1),
-            "int8_TOPs": round(ops / upf / 1e12, 2), "mfma_frac_of_int8_peak": round(ops / upf / 1e12 / 5000.0, 4)}
+            "f16_TFLOPs": round(ops / upf / 1e12, 2), "mfma_frac_of_f16_peak": round(ops / upf / 1e12 / 2500.0, 4)}
         del lp
         torch.cuda.empty_cache()
 
@@ -434,7 +434,7 @@ def main():
             pbytes = ue * eb + sb + E * H * 4 + 2 * T * H * 4
             extra[tag] = {"us_per_chunk": round(upf * 1e6, 2), "tokens_per_s": round(T / upf, 1),
                           "unique_experts": ue, "GBs_unique_weight_bytes": round(pbytes / upf / 1e9, 1),
-                          "int8_TOPs": round(ops / upf / 1e12, 2)}
+                          "f16_TFLOPs": round(ops / upf / 1e12, 2)}
             del lp
             torch.cuda.empty_cache()
 

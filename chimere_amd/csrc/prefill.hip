@@ -225,9 +225,9 @@ __device__ __forceinline__ int excl_scan1024(int v, int* wsum, int* total) {
     return x - v + wsum[w];
 }
 
-// P3: counting sort of the T*K pairs by expert (the order of pairs inside an
-// expert -- by token here -- does not affect any result: every pair's output
-// row is computed on its own), the shared expert as expert E with all T
+// P3: counting sort of the T*K pairs by expert (inside an expert by 16-token top-k
+// work-group, otherwise in any order, which may differ between runs: every
+// pair's output row is computed on its own, so no result depends on it), the shared expert as expert E with all T
 // tokens, and the list of tiles of up to tile_pairs pairs.  Every work-group
 // sums the counts of all top-k work-groups (each expert's total, and what comes
 // before its own PF_PLG of them), scans the totals (thread i: experts 2i and
@@ -376,13 +376,13 @@ static int pf_tile_pairs(int te, int E, int K, int T) {
     return avg <= 13 ? PF_PT : avg <= (te == T_Q8_0 ? 20 : 28) ? 2 * PF_PT : 4 * PF_PT;
 }
 
-// The experts' tiles (at most) above which whole tiles are dealt to the XCDs
+// The experts' tiles (at most) from which whole tiles are dealt to the XCDs
 // (by whole tiles an XCD has at most 12 / tiles more than the average).  Whole /
 // slices (us), H = 2048, F = 512, 256 experts, top-8: 343 tiles IQ3_S + Q5_K 248 / 243;
 // 384 Q4_0 193.1 / 193.6; 408 Q4_0 + Q6_K 235 / 223, IQ3_S + Q5_K 239 / 228, Q4_0
 // 205 / 209; 464 IQ3_S + Q5_K 216 / 218, Q4_0 186 / 189, Q4_0 + Q6_K 195 / 199; 768
 // IQ3_S + Q5_K 808 / 822, Q4_0 733 / 747
-constexpr int PF_WHOLE_TILES = 432;
+constexpr int PF_WHOLE_TILES = 384;
 // Work-groups that the down launch would have at most (the tiles' bound) with two
 // slices each, up to which it takes one: two leave CUs idle behind the longest
 // chain of slices.  Chunk with two / one (us): H = F = 1024, 32 experts, top-2,
@@ -404,7 +404,7 @@ static PfPlan plan_pf(int te, int H, int F, int E, int K, int T) {
     auto tiles = [&](int tp) { return T * K / tp + (T * K < E ? T * K : E); };
     p.max_tiles = tiles(p.tile_pairs);
     p.nsh = (T + p.tile_pairs - 1) / p.tile_pairs;
-    p.whole = p.max_tiles > PF_WHOLE_TILES;
+    p.whole = p.max_tiles >= PF_WHOLE_TILES;
     p.dn_ns = (int64_t)(p.max_tiles + p.nsh) * (H / (2 * PF_ROWS)) <= (F > 256 ? PF_DN_ONE : PF_DN_ONE_K8) ? 1 : 2;
     auto take = [&](size_t& at, size_t bytes) { at = o; o += al256p(bytes); };
     take(p.logits, (size_t)T * E * 4);

@@ -83,9 +83,11 @@ constexpr int pf_cb() { return QTraits<T>::ELEMS == 256 ? QTraits<T>::BYTES : pf
 // any even address (up to 14 bytes into its first granule)
 template <int T>
 constexpr int pf_sl() { return (pf_cb<T>() + 14 + 15) / 16 + (T == T_IQ3_S || T == T_Q6_K || T == T_Q5_K ? 1 : 0); }
-// LDS offset of row r.  An odd number of slots puts 8 consecutive rows on
-// different banks (IQ3_S 9, Q6_K 15, Q5_K 13); 10 slots (Q4_0, Q8_0, Q4_K) do
-// with one slot more after every fourth row.
+// LDS offset of row r.  An odd number of slots starts 8 consecutive rows in
+// different eighths of the banks (IQ3_S 9, Q6_K 15, Q5_K 13); 10 slots (Q4_0, Q8_0, Q4_K) do
+// with one slot more after every fourth row.  (The gate/up profiles still count 0.44 of
+// the LDS cycles in conflict with Q4_0, 0.54 with IQ3_S; besides the codebook
+// lookups it is not known which reads these are.)
 template <int T>
 constexpr bool pf_skew() { return pf_sl<T>() % 2 == 0; }
 template <int T>
@@ -289,7 +291,7 @@ template <> struct PfRow<T_Q6_K> {
     }
 };
 
-// ---- LDS of one work-group: two stages of the weight rows' chunks, of the
+// ---- LDS of one work-group: nw stages (1 or 2) of the weight rows' chunks, two of the
 // activation blocks (units of 8 pairs x 2 blocks) and of their scales
 // ([pair][block]; K-quants also d_x * sum q_x)
 struct PfLds {
@@ -554,7 +556,9 @@ __device__ __forceinline__ void pf_gemm(const PfLds& L, const uint8_t* w0, const
 // which hides a chunk's copies better than a second stage (512 tokens Q4_0
 // gate/up 110 -> 104 us, down 61 -> 55; IQ3_S + Q5_K gate/up 128 -> 117).  16
 // pairs have three work-groups with two stages (one: 45 tokens IQ3_S + Q5_K
-// 76 -> 82 us), 64 pairs two either way, by their registers.  Not for the down
+// 76 -> 82 us), but two where the types are IQ3_S and Q4_0 / Q8_0 (the wider stage
+// of the one and the codebook of the other: 54,816 bytes); 64 pairs two either
+// way, by their registers.  Not for the down
 // launch next to a shared type of two-part blocks: its loop holds up to 199
 // registers, and in a third of the register file Q4_K / Q5_K / Q6_K spilled 25 /
 // 34 / 36 of them (512 tokens, one stage / two: Q4_0 + Q6_K 219 / 203 us, Q4_0 +

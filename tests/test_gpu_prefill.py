@@ -1,5 +1,5 @@
-"""GPU parity of the prefill MoE chunk (chimere_moe_prefill: int8 matrix-core
-grouped GEMMs) against the CPU oracle, through the C ABI.
+"""GPU parity of the prefill MoE chunk (chimere_moe_prefill: grouped GEMMs on the
+matrix cores) against the CPU oracle, through the C ABI.
 
 Bar: routing indices and weights bit-exact; per-token outputs bit-exact
 against the oracle in the prefill order (L=1: one accumulator per row,
@@ -73,9 +73,8 @@ def test_prefill_small(dev, et, st, gate_vec, K, E, T):
     (O.Q4_0, O.IQ3_S, True),
 ])
 def test_prefill_aligned_rows(dev, et, st, gate_vec):
-    """H = 2048: 880-byte IQ3_S rows are 16-byte aligned, so the gate/up GEMM
-    runs the two-stage aligned-span path; 37 tokens leave partially filled
-    16-pair tiles."""
+    """H = 2048: 880-byte IQ3_S and 1152-byte Q4_0 rows, 16-byte aligned ones;
+    37 tokens leave partially filled 16-pair tiles."""
     print(f"prefill aligned et={et} st={st} gate={gate_vec}", flush=True)
     layer = build(dev, 400 + et + st, H=2048, F=512, E=64, K=8, et=et, st=st, gate_vec=gate_vec)
     g = torch.Generator(device=dev).manual_seed(37)
@@ -88,7 +87,7 @@ def test_prefill_iq3s_down_spans(dev, et, st):
     row; each row chunk starts at (440 r + 110 c) % 16 = 0, 2, ..., 14 bytes
     past a 16-byte boundary, so the down's per-row 16-byte span copies place
     it at every even offset of its LDS row (H = 512: the gate/up's 220-byte
-    rows, not 16-byte aligned, take the one-stage path's row staging)."""
+    rows are not 16-byte aligned either)."""
     print(f"prefill iq3s down spans et={et} st={st}", flush=True)
     layer = build(dev, 500 + et + st, H=512, F=1024, E=32, K=4, et=et, st=st, gate_vec=True)
     g = torch.Generator(device=dev).manual_seed(41)
@@ -98,9 +97,8 @@ def test_prefill_iq3s_down_spans(dev, et, st):
 def test_prefill_config5_512(dev):
     """512 tokens, H=2048, F=512, E=256, top-8, Q4_0 experts + Q4_0 shared:
     every token's output, index and weight bit-exact against the oracle.  All
-    256 experts are selected, so every expert's tiles -- the 16-pair tiles of
-    its tokens and its partly filled last tile -- are held to the oracle's
-    bits."""
+    256 experts are selected, so every expert's tiles -- full 32-pair ones and
+    its partly filled last one -- are held to the oracle's bits."""
     layer = build(dev, 5)
     g = torch.Generator(device=dev).manual_seed(55)
     x = torch.randn(512, 2048, generator=g, device=dev)
@@ -215,9 +213,8 @@ def test_prefill_kquant_shared_small(dev, et, st, H, F, E, K, T):
 def test_prefill_q6k_shared_full_shape(dev):
     """A Q6_K shared expert (two int8 scales per 32-element block: the two
     16-element halves in separate products, combined exactly before the
-    block's one rescale) at the model shape: 1680-byte gate/up rows on the
-    two-stage path, 420-byte down rows on the one-stage path, every token
-    bit-exact against the oracle's L=1 order."""
+    block's one rescale) at the model shape: 1680-byte gate/up rows,
+    420-byte down rows (not 16-byte aligned), every token bit-exact against the oracle's L=1 order."""
     print("prefill IQ3_S + Q6_K shared, full shape, 40 tokens", flush=True)
     layer = kq_layer(dev, 890, O.IQ3_S, O.Q6_K, 2048, 512, 256, 8)
     g = torch.Generator(device=dev).manual_seed(89)
