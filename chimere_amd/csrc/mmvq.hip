@@ -413,14 +413,20 @@ static void gemv_entry(const char* who, int type, const void* W, const void* x, 
 // launches / one: Q8_0 4096x2048 (256 work-groups) 5.4 / 4.5 us, Q5_K 5.4 /
 // 4.3; 16384x2048 (1024) Q8_0 10.2 / 9.0, Q4_0 7.9 / 7.1; 65536x2048 (4096)
 // Q4_0 16.1 / 17.7; 8192x4096 (512, two chunks) Q5_K 9.5 / 8.8; 16384x4096
-// (1024, two chunks) Q5_K 12.2 / 13.1.
+// (1024, two chunks) Q5_K 12.2 / 13.1.  Every chunk's quantizing comes before its
+// barrier, so rows of many chunks lose again: 2048x6144 (three chunks) Q8_0 10.1 /
+// 9.9, Q4_K 8.9 / 8.8, Q6_K 10.1 / 11.3; 2048x8192 (four) Q8_0 12.2 / 12.6, Q5_K 11.1
+// / 11.6, Q6_K 12.0 / 14.7.  Not where rows are copied as spans (IQ3_S, Q6_K rows
+// off the 16-byte grid): 2048x7168 IQ3_S 15.5 / 15.0, Q6_K 14.6 / 13.9.
 // Only where the row, the output and the scratch lie apart: the quantizer launch
 // has read all of x before anything is written, so a call may give an output
 // (or, for a short row, a scratch) over its input; in one launch other
 // work-groups still read x when the first ones store.
-static bool f32_one_launch(const float* x, int ncols, int nrows, const float* y, const void* scratch, int ncols_padded) {
+static bool f32_one_launch(int type, const float* x, int ncols, int nrows, const float* y, const void* scratch, int ncols_padded) {
     const int64_t wg = (nrows + TILE_ROWS - 1) / TILE_ROWS, chunks = (ncols + MMVQ_BLOCKS * QK - 1) / (MMVQ_BLOCKS * QK);
-    if (((uintptr_t)x & 15) != 0 || wg * chunks > 1024) return false;   // 16-byte loads of x
+    const bool spans = (type == T_IQ3_S || type == T_Q6_K) && (row_bytes(type, ncols) & 15) != 0;
+    if (wg * chunks > 1024 || (!spans && chunks > (type == T_Q6_K ? 2 : 3))) return false;
+    if (((uintptr_t)x & 15) != 0) return false;   // 16-byte loads of x
     auto apart = [](const void* p, int64_t np, const void* q, int64_t nq) {
         return (uintptr_t)p + (uintptr_t)np <= (uintptr_t)q || (uintptr_t)q + (uintptr_t)nq <= (uintptr_t)p;
     };
@@ -436,7 +442,7 @@ static void gemv_f32_entry(const char* who, int type, const void* W, const float
         return;
     }
     if (!check_gemv(who, type, W, scratch, y, ncols, nrows, ncols_padded / 32, 1)) return;
-    if (f32_one_launch(x, ncols, nrows, y, scratch, ncols_padded)) {
+    if (f32_one_launch(type, x, ncols, nrows, y, scratch, ncols_padded)) {
         MmvqArgs a{(const uint8_t*)W, (const uint8_t*)x, y, ncols, nrows, 1, 0, nrows, nullptr, 0, 0, 0,
                    (uint8_t*)scratch, ncols_padded / 32};
         launch_mmvq_f32(type, a, s);

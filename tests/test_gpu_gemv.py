@@ -407,3 +407,25 @@ def test_f32_gemv_scratch_over_row_or_output(dev, where):
         lib().chimere_mmvq_q8_0_f32(C.c_void_p(w.data_ptr()), p[0], p[1], n, nrows, pad, p[2], G._stream())
         check()
         assert (host(buf[yo:yo + nrows]).view(np.uint32) == want.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("t", [O.Q8_0, O.Q6_K, O.IQ3_S])
+@pytest.mark.parametrize("ncols", [4096, 6144, 7168, 8192])
+def test_f32_gemv_many_chunks(dev, t, ncols):
+    """Rows on both sides of the f32 entry points' lines (one launch up to two or
+    three chunks, any number for rows off the 16-byte grid): the bits of
+    the quantizer launch and the GEMV."""
+    print(f"f32 many chunks type={t} ncols={ncols}", flush=True)
+    rng = np.random.default_rng(ncols + t)
+    nrows = 100
+    w = dev_t(O.quantize(t, rng.normal(0, 0.02, (nrows, ncols)).astype(np.float32)) if t != O.Q6_K
+              else npref.rand_kq(t, nrows, ncols, rng), dev)
+    x = dev_t(rng.standard_normal(ncols).astype(np.float32), dev)
+    fn = {O.Q8_0: G.ggml_gpu_gemv_q8_0_f32, O.Q6_K: G.ggml_gpu_gemv_q6k_f32, O.IQ3_S: G.ggml_gpu_gemv_iq3s_f32}[t]
+    scratch, xq = (torch.full((G.q8_1_row_bytes(ncols),), 7, dtype=torch.uint8, device=dev) for _ in range(2))
+    y, y2 = torch.zeros(nrows, device=dev), torch.zeros(1, nrows, device=dev)
+    fn(w, x, y, scratch, nrows, ncols)
+    G.ggml_gpu_quantize_q8_1_batched(x, xq, ncols, 1)
+    G.gemv_multi(t, w, xq, y2, nrows, ncols, 1)
+    assert (host(y).view(np.uint32) == host(y2)[0].view(np.uint32)).all()
+    assert (host(scratch) == host(xq)).all()
