@@ -322,8 +322,9 @@ static void launch_t(const MmvqArgs& a, int nslots, hipStream_t s) {
         // k_mmvq_tok, 151936x2048) 2 tokens Q4_0 30.8 / 39.5, Q6_K 54 / 57; 3
         // tokens Q5_K 47.3 / 48.5; 4 tokens Q4_0 42.7 / 36.7, Q6_K 66 / 55; 5
         // tokens Q4_0 53 / 57, Q5_K 60 / 77; 8 tokens Q8_0 133 / 84, Q4_0 69 /
-        // 58, Q5_K 85 / 77, Q6_K 106 / 83, IQ3_S 80 / 64, MXFP4 74 / 61; the
-        // K-quants with a min term break even at seven
+        // 58, Q5_K 95 / 86, Q6_K 106 / 83, IQ3_S 80 / 64, MXFP4 74 / 61; 7
+        // tokens Q4_K 71.8 / 70.4, Q5_K 77 / 85 (16384x4096 21.7 / 23.5, but 4096x2048,
+        // one work-group per CU, 8.7 / 8.3)
         constexpr bool KQ = T == T_Q4_K || T == T_Q5_K;
         switch (a.ntok) {
         case 1: hipLaunchKernelGGL((k_mmvq<T, 1>), grid, blk, 0, s, a); break;
@@ -336,6 +337,13 @@ static void launch_t(const MmvqArgs& a, int nslots, hipStream_t s) {
                 hipLaunchKernelGGL((k_mmvq<T, 6>), grid, blk, 0, s, a);
                 break;
             }
+            [[fallthrough]];
+        case 7:
+            if constexpr (T == T_Q5_K)
+                if (a.ntok == 7 && grid.x > 256) {
+                    hipLaunchKernelGGL((k_mmvq<T, 7>), grid, blk, 0, s, a);
+                    break;
+                }
             [[fallthrough]];
         default: hipLaunchKernelGGL((k_mmvq_tok<T, 2>), grid, blk, 0, s, a); break;
         }

@@ -429,3 +429,19 @@ def test_f32_gemv_many_chunks(dev, t, ncols):
     G.gemv_multi(t, w, xq, y2, nrows, ncols, 1)
     assert (host(y).view(np.uint32) == host(y2)[0].view(np.uint32)).all()
     assert (host(scratch) == host(xq)).all()
+
+
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K])
+@pytest.mark.parametrize("nrows", [4096, 4099])
+def test_seven_tokens_both_kernels(dev, t, nrows):
+    """Seven tokens of the types with a min term, with one work-group per CU and
+    with one more (Q5_K: the matrix-core kernel, the other one): bit-exact
+    against the oracle."""
+    print(f"seven tokens type={t} nrows={nrows}", flush=True)
+    rng = np.random.default_rng(nrows + t)
+    w = npref.rand_kq(t, nrows, 512, rng)
+    xq = O.quantize_q8_1(rng.standard_normal((7, 512)).astype(np.float32))
+    y = torch.zeros(7, nrows, device=dev)
+    G.gemv_multi(t, dev_t(w, dev), dev_t(xq, dev), y, nrows, 512, 7)
+    yo = O.gemv(t, w, xq, 512, nrows, ntok=7, xq_stride=xq.shape[1])
+    assert (host(y).view(np.uint32) == np.asarray(yo).reshape(7, nrows).view(np.uint32)).all()
